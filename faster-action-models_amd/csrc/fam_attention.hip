@@ -1154,7 +1154,7 @@ __global__ __launch_bounds__(256) void attn_cross_kernel(AttnArgs a) {
 }
 
 // ---------------------------------------------------------------------------------------
-// attn_long_kernel: long query sequences (video tokens), one key segment, no mask or a key mask.
+// attn_long_kernel: long query sequences (video tokens), one key segment, no mask or a boolean one.
 // A workgroup of 4 waves owns 128 queries of one (batch, head), 32 per wave; keys stream in
 // 64-key tiles through double-buffered LDS (K and V row-major), one barrier per tile, the
 // next tile's buffer loads in flight during the current tile's math.  Per wave and tile:
@@ -1168,15 +1168,23 @@ __global__ __launch_bounds__(256) void attn_cross_kernel(AttnArgs a) {
 // At most 256 registers per lane, so two workgroups share a CU and one's vector work fills
 // the other's matrix-core gaps.  Work-groups are mapped so that all query blocks of one head
 // run on the same XCD (its 4 MB L2 then holds that head's K/V once).
-// KMASK: a boolean key mask shared by every query (mask query stride 0: the text padding mask
+// MK = 1: a boolean key mask shared by every query (mask query stride 0: the text padding mask
 // of the cross-attention, [B, Lc] or [B, H, Lc]); each tile's 64 entries travel with the K/V
 // tile as additive 0 / -inf terms in LDS (keys past Sk included).
+// MK = 2: a boolean mask with rows of its own for every query (the first-frame-causal video mask,
+// the joint [video ; action] mask).  The lane that owns query q with keys 4 hh + 8 g .. + 3 of a
+// half-tile reads 32 contiguous bytes of row q (keys 32 hh .. + 31 of the tile, any alignment) and
+// trades every other dword with lane l ^ 32, so a tile costs a lane two 16-byte loads; they are in
+// flight under the softmax and P V of the tile before.  A wave none of whose 32 x 64 entries is set
+// leaves the tile's products out, one with all of them set skips the selects.  1592 x 1592 joint
+// mask, 24 x 128 heads: 273 us on attn_tiled_kernel, 60.5 us here.
 // KW = 2 (head dim 128, a grid of at most one workgroup per CU): 8 waves in two key groups of
 // 4; group g takes the tiles g, g + 2, g + 4, ... of the same 128 queries with its own LDS slots,
 // so each SIMD runs two waves (one's softmax under the other's MFMAs) although the grid leaves
 // one workgroup per CU, and group 1 hands its softmax state to group 0 through LDS at the end.
-template <int DH, bool KMASK, int KW>
+template <int DH, int MK, int KW>
 __global__ __launch_bounds__(256 * KW, 2 / KW) void attn_long_kernel(AttnArgs a, int nqb) {
+  constexpr bool KMASK = MK == 1, QMASK = MK == 2;
   constexpr int NTH = 256 * KW;          // threads; 32 queries per wave, KW waves per query group
   constexpr int BN = 64;                 // keys per tile
   constexpr int KS = DH / 16;            // 16-wide k-steps of S^T = K Q^T
@@ -1291,6 +1299,31 @@ __global__ __launch_bounds__(256 * KW, 2 / KW) void attn_long_kernel(AttnArgs a,
       if (gtid < BN) Mb[buf][kg][gtid] = mr ? 0.f : -INFINITY;
     }
   };
+  // per-query mask bytes of tile t: keys 32 hh .. + 31 of the tile of this lane's query (0 past Sk)
+  const uint8_t* mq = QMASK ? reinterpret_cast<const uint8_t*>(a.mask) + b * a.mbs + h * a.mhs + (int64_t)qc * a.mqs
+                            : nullptr;
+  uint32_t mw[QMASK ? 8 : 1];
+  auto gload_q = [&](int t) {
+    if constexpr (QMASK) {
+      const int k0 = t * BN + 32 * hh;
+      if (t * BN + BN <= Sk) {   // uniform
+        __builtin_memcpy(&mw[0], mq + k0, 16);
+        __builtin_memcpy(&mw[4], mq + k0 + 16, 16);
+      } else {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          uint32_t w = 0;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const int key = k0 + 4 * j + e;
+            const uint32_t v = mq[key < Sk ? key : 0];
+            w |= (key < Sk && v ? 1u : 0u) << (8 * e);
+          }
+          mw[j] = w;
+        }
+      }
+    }
+  };
   // A operand of the PV product (V^T: row = dim, k = key) straight from the row-major tile
   // with two transposing LDS reads (ds_read_b64_tr_b16).  Within each 16-lane group, lane i
   // receives element i % 4 of the 8-byte loads of lanes i / 4 + 4e (e = 0..3); so lane s of a
@@ -1343,7 +1376,7 @@ __global__ __launch_bounds__(256 * KW, 2 / KW) void attn_long_kernel(AttnArgs a,
   float m_run = -INFINITY, l_run = 0.f;
   const float sl2 = a.scale_log2;
   const int ntiles_kw = (Sk + BN - 1) / BN;
-  const int nfull_kw = KMASK ? ntiles_kw : Sk / BN;
+  const int nfull_kw = MK ? ntiles_kw : Sk / BN;
 
   // one 64-key tile t of this key group from LDS buffer BUF; TAIL (the partial last tile
   // without a key mask) sets the scores of keys past Sk to -inf, so full tiles carry no
@@ -1352,6 +1385,22 @@ __global__ __launch_bounds__(256 * KW, 2 / KW) void attn_long_kernel(AttnArgs a,
   auto compute = [&](int t, auto tail_tag, auto buf_tag) {
     constexpr bool TAIL = decltype(tail_tag)::value;
     constexpr int buf = decltype(buf_tag)::value;
+    bool some = false;
+    if constexpr (QMASK) {
+      // (X, Y) = (dword 2g, dword 2g + 1) of keys 32 hh ..: the swap leaves dword 2g + hh of the
+      // first half-tile in X and of the second in Y.  A byte is any non-zero value.
+      uint32_t lo = 0, all = 0x01010101u;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        lo |= mw[j];
+        all &= mw[j];
+      }
+      if (!__any(lo != 0)) {
+        gload_q(t + KW);
+        return;
+      }
+      some = __any(all != 0x01010101u);
+    }
     f32x16 st[2] = {f32x16{}, f32x16{}};
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks)
@@ -1367,6 +1416,19 @@ __global__ __launch_bounds__(256 * KW, 2 / KW) void attn_long_kernel(AttnArgs a,
 #pragma unroll
           for (int e = 0; e < 4; ++e) st[kt][4 * g4 + e] += m4[e];
         }
+    } else if constexpr (QMASK) {
+      if (some) {
+#pragma unroll
+        for (int g4 = 0; g4 < 4; ++g4) {
+          const auto sw = __builtin_amdgcn_permlane32_swap(mw[2 * g4], mw[2 * g4 + 1], false, false);
+#pragma unroll
+          for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              st[kt][4 * g4 + e] = (sw[kt] >> (8 * e)) & 0xffu ? st[kt][4 * g4 + e] : -INFINITY;
+        }
+      }
+      gload_q(t + KW);
     } else if constexpr (TAIL) {
       const int kleft = Sk - t * BN - 4 * hh;   // keys of this tile below Sk, relative to the lane's first
 #pragma unroll
@@ -1387,14 +1449,15 @@ __global__ __launch_bounds__(256 * KW, 2 / KW) void attn_long_kernel(AttnArgs a,
     const float mloc = mraw * sl2;   // sl2 > 0
     if (__any(mloc > m_run + 8.0f)) {
       const float m_new = fmaxf(m_run, mloc);
-      const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);   // max unchanged: 1; -inf: 0
+      // max unchanged: 1; -inf: 0 (a query of its own mask rows may still have no key: -inf - -inf)
+      const float alpha = __builtin_amdgcn_exp2f(m_run - (QMASK && m_new == -INFINITY ? 0.f : m_new));
       l_run *= alpha;
 #pragma unroll
       for (int d = 0; d < DT; ++d) acc[d] *= alpha;
       m_run = m_new;
     }
     // (a query whose keys so far are all masked keeps m_run = -inf: its p are exp2(-inf) = 0)
-    const float m_use = KMASK && m_run == -INFINITY ? 0.f : m_run;
+    const float m_use = MK && m_run == -INFINITY ? 0.f : m_run;
     float psum = 0.f;
     bf16x8 pf[2][2];
 #pragma unroll
@@ -1446,6 +1509,7 @@ __global__ __launch_bounds__(256 * KW, 2 / KW) void attn_long_kernel(AttnArgs a,
 
   const int ntiles = ntiles_kw;
   const int nfull = nfull_kw;   // tiles whose keys are all below Sk (or masked)
+  gload_q(kg);
   prefetch(kg, 0);
   finish(0);
   using F = std::false_type;
@@ -1779,8 +1843,8 @@ static void launch_dh(const AttnArgs& a, int64_t bh, hipStream_t s) {
     if constexpr (DH == 64 || DH == 128) {
       // (buffer loads address a head's K and V rows with 32-bit byte offsets)
       const bool fits32 = a.Sk * a.k0_rs * 2 < ((int64_t)1 << 31) && a.Sk * a.v0_rs * 2 < ((int64_t)1 << 31);
-      const bool kmask = a.mask_kind == FAM_MASK_BOOL && a.mqs == 0;
-      if (a.sk0 == a.Sk && (a.mask_kind == FAM_MASK_NONE || kmask) && a.Sk >= 1 && fits32 && a.k0_rs >= DH &&
+      const int mk = a.mask_kind == FAM_MASK_NONE ? 0 : (a.mqs == 0 ? 1 : 2);
+      if (a.sk0 == a.Sk && (a.mask_kind == FAM_MASK_NONE || a.mask_kind == FAM_MASK_BOOL) && a.Sk >= 1 && fits32 && a.k0_rs >= DH &&
           a.v0_rs >= DH) {
         const int nqb = (int)((a.Sq + 127) / 128);
         const dim3 grid((unsigned)(nqb * bh));
@@ -1788,13 +1852,15 @@ static void launch_dh(const AttnArgs& a, int64_t bh, hipStream_t s) {
         // (two waves per SIMD); more workgroups share the CUs two by two instead
         if constexpr (DH == 128) {
           if (nqb * bh <= fam_host::device_cus()) {
-            if (kmask) FAM_LAUNCH((attn_long_kernel<DH, true, 2>), grid, dim3(512), 0, s, a, nqb);
-            else FAM_LAUNCH((attn_long_kernel<DH, false, 2>), grid, dim3(512), 0, s, a, nqb);
+            if (mk == 1) FAM_LAUNCH((attn_long_kernel<DH, 1, 2>), grid, dim3(512), 0, s, a, nqb);
+            else if (mk == 2) FAM_LAUNCH((attn_long_kernel<DH, 2, 2>), grid, dim3(512), 0, s, a, nqb);
+            else FAM_LAUNCH((attn_long_kernel<DH, 0, 2>), grid, dim3(512), 0, s, a, nqb);
             return;
           }
         }
-        if (kmask) FAM_LAUNCH((attn_long_kernel<DH, true, 1>), grid, dim3(256), 0, s, a, nqb);
-        else FAM_LAUNCH((attn_long_kernel<DH, false, 1>), grid, dim3(256), 0, s, a, nqb);
+        if (mk == 1) FAM_LAUNCH((attn_long_kernel<DH, 1, 1>), grid, dim3(256), 0, s, a, nqb);
+        else if (mk == 2) FAM_LAUNCH((attn_long_kernel<DH, 2, 1>), grid, dim3(256), 0, s, a, nqb);
+        else FAM_LAUNCH((attn_long_kernel<DH, 0, 1>), grid, dim3(256), 0, s, a, nqb);
         return;
       }
     }

@@ -920,6 +920,41 @@ def test_attention_long_sequences(B, H, Sq, Sk, Dh):
     assert relerr(y, ref) <= TOL
 
 
+@pytest.mark.parametrize("B,H,Sq,Sk,Dh,kind", [(1, 2, 70, 300, 128, "joint"), (2, 3, 200, 333, 64, "random"),
+                                                (1, 24, 1592, 1592, 128, "joint"), (2, 3, 257, 320, 128, "random"),
+                                                (1, 24, 1430, 270, 128, "random"), (1, 2, 129, 257, 128, "odd"),
+                                                (2, 2, 130, 258, 64, "odd"), (1, 2, 100, 258, 128, "random")])
+def test_attention_long_query_mask(B, H, Sq, Sk, Dh, kind):
+    """A bool mask with a row per query on the long kernel: the joint [video ; action] mask (tiles that are
+    all set, all clear and mixed for a wave), random masks with a fully masked query (zeros out) and a first
+    tile masked for one query; an odd row pitch at an odd address ("odd": a column window of a wider mask), a
+    partial last tile, one and two key groups.  The bar is the file's 2e-2 of the largest value; what may
+    differ is the rounding of the probabilities to bf16 (2^-9 each)."""
+    q, k, v = rnd(B, Sq, H * Dh, seed=161), rnd(B, Sk, H * Dh, seed=162), rnd(B, Sk, H * Dh, seed=163)
+    g = torch.Generator().manual_seed(164)
+    if kind == "joint":
+        first, action = Sk // 2 - 16, 32
+        mask = torch.zeros(Sq, Sk, dtype=torch.bool)
+        mask[:Sq - action, :Sk - action] = True
+        mask[:first, first:] = False
+        mask[Sq - action:, Sk - action:] = True
+        mask[Sq - action:, :first] = True
+        mask_d = dev(mask)
+    else:
+        wide = torch.rand(B, 1, Sq, Sk + 7, generator=g) > 0.6
+        wide[:, :, 3] = False
+        wide[:, :, 5, :80] = False
+        wide[:, :, 64:] |= torch.rand(B, 1, Sq - 64, 1, generator=g) > 0.5   # rows with every key set
+        wide = wide if kind == "odd" else wide[..., 3:3 + Sk].contiguous()
+        off = 3 if kind == "odd" else 0
+        mask, mask_d = wide[..., off:off + Sk], dev(wide)[..., off:off + Sk]
+    ref = O.flash_attention(q.float(), k.float(), v.float(), H, mask)
+    y = ops().flash_attention(dev(q), dev(k), dev(v), H, ctx_mask=mask_d)
+    assert relerr(y, ref) <= TOL
+    if kind != "joint":
+        assert torch.all(y[:, 3] == 0)
+
+
 # --------------------------------------------------------------------------- rows past the end
 def _nan_tailed(rows, cols, pad, seed, scale=1.0):
     """[rows + pad, cols] bf16 whose first `rows` rows are N(0, scale) and the rest NaN: a view of
