@@ -202,6 +202,57 @@ __device__ __forceinline__ void row_stats(const GemmArgs& g, int64_t m0, int row
 }
 
 // ---------------------------------------------------------------------------------------
+// Staged operand panels (M <= 64): a wave's MFMA fragment of 16 rows x 32 k, loaded straight from
+// row-major memory, is 16 separate 64-byte pieces, and a launch that loads 100 KB of them per CU
+// waits on its address processing, not on memory (M = 32, K = 1024, graph-timed: 4.8 us with the
+// weights in HBM, 4.5 us with everything in L2, 1.8 us for a kernel that only loads and stores).
+// A staged wave fetches the KW-wide k range that it alone uses, of every row, with direct-to-LDS
+// buffer loads instead: one load is 1 KB = 512 / KW rows of KW contiguous values.  Nothing is
+// shared between waves, so the wave's own vmcnt wait is all the synchronisation there is before
+// its products.  The 16-byte chunk c of row r sits at c ^ panel_swz(r) (lane j fetches the chunk
+// that belongs in its slot), which makes the fragment reads of 16 rows hit 16 distinct bank
+// groups.  Rows past M or N are past the descriptor's range and read zeros.
+template <int KW>
+__device__ __forceinline__ int panel_swz(int r) { return KW == 64 ? (r >> 1) & 7 : r & 15; }
+
+// ROWS rows (a multiple of 16) of the panel at byte column kb; lds and kb are wave-uniform
+template <int KW, int ROWS>
+__device__ __forceinline__ void panel_stage(__amdgpu_buffer_rsrc_t rs, uint32_t ld2, uint32_t kb, bf16* lds, int lane) {
+  constexpr int CPR = KW / 8, RPI = 512 / KW;   // chunks per row, rows per load
+  static_assert(KW == 64 || KW == 128 || KW == 256, "panel width");
+  const int lr = lane / CPR, lc = lane % CPR;
+#pragma unroll
+  for (int i = 0; i < ROWS / RPI; ++i) {
+    const int r = i * RPI + lr;
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void*)(lds + i * 512), 16,
+                                             (uint32_t)r * ld2 + kb + (uint32_t)((lc ^ panel_swz<KW>(r)) * 16), 0, 0, 0);
+  }
+}
+// the fragment of rows r0 .. r0 + 15 (r0 a multiple of 16), k-step s
+template <int KW>
+__device__ __forceinline__ bf16x8 panel_frag(const bf16* lds, int r0, int s, int l16, int lg) {
+  return *reinterpret_cast<const bf16x8*>(lds + (r0 + l16) * KW + (((4 * s + lg) ^ panel_swz<KW>(l16)) * 8));
+}
+// this wave's staged loads have landed in its own panel (its ds reads may follow); the empty asm
+// statements keep LDS reads and writes from moving across
+__device__ __forceinline__ void panel_wait() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt(0x0070);   // vmcnt(0) lgkmcnt(0)
+  asm volatile("" ::: "memory");
+}
+// one wave's product over its KW of K: acc[t] = W (16 x KW) A_t^T.  WD: the weight panel straight
+// into registers (wf, loaded by the caller) where a staged one would not fit the LDS
+template <int MT, int KW, bool WD>
+__device__ __forceinline__ void panel_mfma(const bf16* lds, const bf16x8* wf, int l16, int lg, f32x4 (&acc)[MT]) {
+#pragma unroll
+  for (int s = 0; s < KW / 32; ++s) {
+    const bf16x8 w = WD ? wf[s] : panel_frag<KW>(lds, 16 * MT, s, l16, lg);
+#pragma unroll
+    for (int t = 0; t < MT; ++t) acc[t] = mfma16(w, panel_frag<KW>(lds, 16 * t, s, l16, lg), acc[t]);
+  }
+}
+
+// ---------------------------------------------------------------------------------------
 // skinny_kernel: M <= 16*MT rows, 16 output columns per workgroup, NW waves split K into
 // contiguous runs of 32-wide k-steps; each wave holds KS k-steps of weights and activations
 // in registers at once.  Every load is branch-free (out-of-range lanes load a valid address
@@ -496,6 +547,59 @@ __global__ __launch_bounds__(256) void partial_kernel(PartArgs g) {
   }
 }
 
+// partial_staged_kernel: partial_kernel's split (16 columns x 4 KW of K per workgroup, the same
+// planes) with staged panels.  K is a multiple of KW: a wave's range lies in K or past it.
+// Measured at M = 32, N = 1024 (graph-timed, weights from HBM): K = 1024 in 4 planes 2.7 -> 2.4
+// us, K = 4096 in 4 planes 5.3 -> 4.15 us.
+template <int MT, int KW>
+__global__ __launch_bounds__(256) void partial_staged_kernel(PartArgs g) {
+  constexpr bool WD = MT == 4 && KW == 256;   // 4 x 80 rows x 512 B would be the whole LDS
+  constexpr int ROWS = 16 * MT + (WD ? 0 : 16);
+  __shared__ __attribute__((aligned(1024))) bf16 sm[4][ROWS * KW];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l16 = lane & 15, lg = lane >> 4;
+  const int M = (int)g.M, N = (int)g.N, K = (int)g.K;
+  const int n0 = blockIdx.x * 16, z = blockIdx.y, k0 = (z * 4 + wave) * KW;
+  f32x4 acc[MT];
+#pragma unroll
+  for (int t = 0; t < MT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  if (k0 < K) {
+    const uint32_t lda2 = (uint32_t)g.lda * 2u, ldw2 = (uint32_t)g.ldw * 2u, kb = (uint32_t)k0 * 2u;
+    const auto rw = buffer_rsrc(g.w + (int64_t)n0 * g.ldw, (uint32_t)min(16, N - n0) * ldw2);
+    bf16x8 wf[WD ? KW / 32 : 1];
+    if constexpr (WD) {
+#pragma unroll
+      for (int s = 0; s < KW / 32; ++s) wf[s] = buffer_load8(rw, (uint32_t)l16 * ldw2 + kb + (uint32_t)(4 * s + lg) * 16u);
+    } else {
+      panel_stage<KW, 16>(rw, ldw2, kb, &sm[wave][16 * MT * KW], lane);
+    }
+    panel_stage<KW, 16 * MT>(buffer_rsrc(g.a, (uint32_t)M * lda2), lda2, kb, &sm[wave][0], lane);
+    panel_wait();
+    panel_mfma<MT, KW, WD>(&sm[wave][0], wf, l16, lg, acc);
+  }
+  // the wave accumulators meet in the waves' own panels
+  asm volatile("" ::: "memory");
+#pragma unroll
+  for (int t = 0; t < MT; ++t) *reinterpret_cast<f32x4*>(&sm[wave][(t * 64 + lane) * 8]) = acc[t];
+  __syncthreads();
+  for (int t = wave; t < MT; t += 4) {
+    f32x4 r[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) r[q] = *reinterpret_cast<const f32x4*>(&sm[q][(t * 64 + lane) * 8]);
+    const f32x4 v = ((r[0] + r[1]) + r[2]) + r[3];
+    const int m = t * 16 + l16, n = n0 + lg * 4;
+    if (m >= M) continue;
+    float* dst = g.part + ((int64_t)z * M + m) * N + n;
+    if ((N & 3) == 0) {
+      if (n < N) *reinterpret_cast<f32x4*>(dst) = v;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (n + e < N) dst[e] = v[e];
+    }
+  }
+}
+
 // ---------------------------------------------------------------------------------------
 // partial_wide_kernel (64 < M <= 128: the video prefill's 98-token projections; M <= 64 with
 // two strips for the large action projections, see partial_plan): the same
@@ -702,6 +806,34 @@ struct FinalArgs {
   int64_t M, N, K;
 };
 
+// the epilogue of one m-tile: v = the product's 4 columns nc .. nc + 3 of row m
+__device__ __forceinline__ void final_store(const FinalArgs& g, int64_t m, int64_t nc, int lg, f32x4 v, const float (&bias)[4]) {
+  bf16x4 o;
+  float ss = 0.f;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    float x = v[e] + bias[e];
+    if (g.act == FAM_ACT_GELU_TANH) x = gelu_tanh(x);
+    else if (g.act == FAM_ACT_SILU) x = silu(x);
+    else if (g.act == FAM_ACT_RELU) x = fmaxf(x, 0.f);
+    else if (g.act == FAM_ACT_GELU_ERF) x = gelu_erf(x);
+    o[e] = to_bf(x);
+    const float r = to_f(o[e]);
+    ss += (nc + e < g.N) ? r * r : 0.f;
+  }
+  ss = group4_sum(ss);  // the 16 columns of this group, fixed order
+  if (m >= g.M) return;
+  bf16* dst = g.out + m * g.ldo + nc;
+  if ((g.N & 3) == 0 && (g.ldo & 3) == 0) {
+    if (nc < g.N) *reinterpret_cast<bf16x4*>(dst) = o;
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (nc + e < g.N) dst[e] = o[e];
+  }
+  if (g.sumsq && lg == 0) g.sumsq[m * (int64_t)gridDim.x + blockIdx.x] = ss;
+}
+
 template <int MT, int NW, int STEPS>
 __global__ __launch_bounds__(NW * 64) void final_kernel(FinalArgs g) {
   __shared__ f32x4 red[NW][MT][64];
@@ -758,31 +890,58 @@ __global__ __launch_bounds__(NW * 64) void final_kernel(FinalArgs g) {
     f32x4 v = red[0][t][lane];
 #pragma unroll
     for (int q = 1; q < NW; ++q) v += red[q][t][lane];
-    const int64_t m = t * 16 + l16;            // D[col = 4*lg + e][row = l16]
-    bf16x4 o;
-    float ss = 0.f;
+    final_store(g, t * 16 + l16, nc, lg, v, bias);   // D[col = 4*lg + e][row = l16]
+  }
+}
+
+// final_staged_kernel: the same workgroup (16 columns, whole K, 4 waves) with staged panels, for
+// K <= 1024, a multiple of KW.  Graph-timed at M = 32, K = 1024 with the weights in HBM: N = 1024
+// 4.8 -> 3.35 us, 3072 5.3 -> 4.15 us, 4096 + GELU 5.6 -> 4.6 us.  A workgroup holds up to 96 KB of
+// LDS (M <= 32; 128 KB at 64 rows), so one runs per CU: also above 256 workgroups ahead of the
+// register form (N = 9216: 10.8 -> 9.1 us for the bare product).
+template <int MT, int KW>
+__global__ __launch_bounds__(256) void final_staged_kernel(FinalArgs g) {
+  constexpr bool WD = MT == 4 && KW == 256;
+  constexpr int ROWS = 16 * MT + (WD ? 0 : 16);
+  __shared__ __attribute__((aligned(1024))) bf16 sm[4][ROWS * KW];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l16 = lane & 15, lg = lane >> 4;
+  const int M = (int)g.M, N = (int)g.N, K = (int)g.K;
+  const int n0 = blockIdx.x * 16, k0 = wave * KW, nc = n0 + lg * 4;
+  f32x4 acc[MT];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      float x = v[e] + bias[e];
-      if (g.act == FAM_ACT_GELU_TANH) x = gelu_tanh(x);
-      else if (g.act == FAM_ACT_SILU) x = silu(x);
-      else if (g.act == FAM_ACT_RELU) x = fmaxf(x, 0.f);
-      else if (g.act == FAM_ACT_GELU_ERF) x = gelu_erf(x);
-      o[e] = to_bf(x);
-      const float r = to_f(o[e]);
-      ss += (nc + e < g.N) ? r * r : 0.f;
-    }
-    ss = group4_sum(ss);  // the 16 columns of this group, fixed order
-    if (m >= g.M) continue;
-    bf16* dst = g.out + m * g.ldo + nc;
-    if ((g.N & 3) == 0 && (g.ldo & 3) == 0) {
-      if (nc < g.N) *reinterpret_cast<bf16x4*>(dst) = o;
+  for (int t = 0; t < MT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // the epilogue's bias, in flight with the panels (no branch: a readable address without one)
+  const bf16* bsrc = g.bias ? g.bias : g.w;
+  bf16 braw[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) braw[e] = bsrc[min(nc + e, N - 1)];
+  if (k0 < K) {
+    const uint32_t lda2 = (uint32_t)g.lda * 2u, ldw2 = (uint32_t)g.ldw * 2u, kb = (uint32_t)k0 * 2u;
+    const auto rw = buffer_rsrc(g.w + (int64_t)n0 * g.ldw, (uint32_t)min(16, N - n0) * ldw2);
+    bf16x8 wf[WD ? KW / 32 : 1];
+    if constexpr (WD) {
+#pragma unroll
+      for (int s = 0; s < KW / 32; ++s) wf[s] = buffer_load8(rw, (uint32_t)l16 * ldw2 + kb + (uint32_t)(4 * s + lg) * 16u);
     } else {
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        if (nc + e < g.N) dst[e] = o[e];
+      panel_stage<KW, 16>(rw, ldw2, kb, &sm[wave][16 * MT * KW], lane);
     }
-    if (g.sumsq && lg == 0) g.sumsq[m * (int64_t)gridDim.x + blockIdx.x] = ss;
+    panel_stage<KW, 16 * MT>(buffer_rsrc(g.a, (uint32_t)M * lda2), lda2, kb, &sm[wave][0], lane);
+    panel_wait();
+    panel_mfma<MT, KW, WD>(&sm[wave][0], wf, l16, lg, acc);
+  }
+  asm volatile("" ::: "memory");
+#pragma unroll
+  for (int t = 0; t < MT; ++t) *reinterpret_cast<f32x4*>(&sm[wave][(t * 64 + lane) * 8]) = acc[t];
+  __syncthreads();
+  float bias[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) bias[e] = g.bias ? to_f(braw[e]) : 0.f;
+  for (int t = wave; t < MT; t += 4) {
+    f32x4 r[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) r[q] = *reinterpret_cast<const f32x4*>(&sm[q][(t * 64 + lane) * 8]);
+    final_store(g, t * 16 + l16, nc, lg, ((r[0] + r[1]) + r[2]) + r[3], bias);
   }
 }
 
@@ -1597,9 +1756,24 @@ extern "C" int fam_gemm_partial_splits(int64_t M, int64_t N, int64_t K) {
   return M > 128 && st >= 0 ? 0 : sp;
 }
 
+// Staged panels address a (M rows) and 16 weight rows with 32-bit byte offsets, and a wave's whole
+// KW-wide range has to lie inside K.
+static bool panel_ok(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldw, int kw) {
+  return K % kw == 0 && M * lda * 2 < (1LL << 31) && ldw < (1LL << 25) && N < (1LL << 31) - 16 && K < (1LL << 30);
+}
+
 template <int MT>
 static void launch_partial(const PartArgs& a, int steps, int splits, hipStream_t s) {
   const dim3 grid((unsigned)((a.N + 15) / 16), (unsigned)splits);
+  if constexpr (MT <= 4) {
+    // (one k-step per wave is a 64-byte piece per row either way)
+    if (steps > 1 && panel_ok(a.M, a.N, a.K, a.lda, a.ldw, 32 * steps)) {
+      if (steps == 2) FAM_LAUNCH((partial_staged_kernel<MT, 64>), grid, dim3(256), 0, s, a);
+      else if (steps == 4) FAM_LAUNCH((partial_staged_kernel<MT, 128>), grid, dim3(256), 0, s, a);
+      else FAM_LAUNCH((partial_staged_kernel<MT, 256>), grid, dim3(256), 0, s, a);
+      return;
+    }
+  }
   switch (steps) {
     case 1: FAM_LAUNCH((partial_kernel<MT, 1>), grid, dim3(256), 0, s, a); break;
     case 2: FAM_LAUNCH((partial_kernel<MT, 2>), grid, dim3(256), 0, s, a); break;
@@ -1717,6 +1891,16 @@ static void launch_final_steps(const FinalArgs& a, int steps, hipStream_t s) {
 
 template <int MT>
 static void launch_final(const FinalArgs& a, hipStream_t s) {
+  // K <= 1024 in whole panels (the narrowest of 64, 128, 256 columns that four waves cover K
+  // with): staged.  Otherwise the register form:
+  const int kw = a.K <= 256 ? 64 : a.K <= 512 ? 128 : 256;
+  if (a.K <= 1024 && panel_ok(a.M, a.N, a.K, a.lda, a.ldw, kw)) {
+    const dim3 grid((unsigned)((a.N + 15) / 16));
+    if (kw == 64) FAM_LAUNCH((final_staged_kernel<MT, 64>), grid, dim3(256), 0, s, a);
+    else if (kw == 128) FAM_LAUNCH((final_staged_kernel<MT, 128>), grid, dim3(256), 0, s, a);
+    else FAM_LAUNCH((final_staged_kernel<MT, 256>), grid, dim3(256), 0, s, a);
+    return;
+  }
   // K <= 1024: 4 waves; longer: 16 waves; k-steps per wave 1, 2, 4 or 8.  Graph-timed at
   // M = 32, K = 1024 (N = 1024 / 3072 / 4096), 4 waves of 8 k-steps beat 8 waves of 4 by
   // 0.1-0.3 us a launch (the 4-way merge of the wave sums is shorter); above K = 1024 the 16

@@ -1001,3 +1001,29 @@ def test_gemm_rows_past_the_end_read_as_zero(M, N, K):
     y = torch.empty(M, N, dtype=torch.bfloat16, device="cuda")
     ops().rowop(y, partials=part, bias=bd)
     assert relerr(y, ref) <= TOL
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 16, 64), (16, 33, 256), (17, 1024, 1024), (32, 1003, 768), (33, 48, 512),
+                                   (64, 1030, 1024), (32, 1024, 4096), (17, 1024, 3072), (31, 520, 1088), (5, 7, 192)])
+def test_staged_panels_small_m(M, N, K):
+    """fam_gemm_partial and fam_gemm_final at <= 64 rows, whose operands reach the MFMAs through LDS panels
+    of 64, 128 or 256 columns per wave: rows and columns that do not fill a 16-row tile, K that leaves waves
+    without a range (768, 192), K outside the panels (1088: the register form), row pitches wider than K with
+    NaN around the operands (a read outside them would show).  fp32 sums of exact bf16 products: within
+    K 2^-23 sum |a| |w| of float64 in any order; the bf16 result adds half an ulp (2^-9)."""
+    a = torch.full((M + 16, K + 64), float("nan"), dtype=torch.bfloat16)
+    w = torch.full((N + 16, K + 64), float("nan"), dtype=torch.bfloat16)
+    a[:M, :K], w[:N, :K] = rnd(M, K, seed=171), rnd(N, K, seed=172, scale=0.02)
+    b = rnd(N, seed=173, scale=0.02)
+    ad, wd = dev(a)[:M, :K], dev(w)[:N, :K]
+    ref = a[:M, :K].double() @ w[:N, :K].double().t()
+    lim = K * 2.0 ** -23 * (a[:M, :K].double().abs() @ w[:N, :K].double().abs().t())
+    part, S = ops().gemm_partial(ad, wd)
+    assert ((part.double().sum(0).cpu() - ref).abs() <= lim).all()
+    if K <= 4096:
+        y, ss = ops().gemm_final(ad, wd, dev(b), want_sumsq=True)
+        y = y.double().cpu()
+        rb = ref + b.double()
+        assert ((y - rb).abs() <= lim + rb.abs() * 2.0 ** -8 + 1e-30).all()
+        sq = torch.nn.functional.pad(y.square(), (0, -N % 16)).reshape(M, -1, 16).sum(-1)
+        assert torch.allclose(ss.double().cpu(), sq, rtol=1e-5, atol=1e-12)
