@@ -467,6 +467,114 @@ __global__ __launch_bounds__(NW * 64) void skinny_kernel(GemmArgs g) {
   }
 }
 
+// skinny_staged_kernel: the same product and epilogue (no prologue, or the folded LayerNorm) with
+// staged panels, NW waves of KW columns covering K (a multiple of KW).  The row sums of the folded
+// form come from the fragments the MFMAs use; it takes 8 waves, so that a SIMD's two waves share
+// them, the plain form 4.  17 rows x 768 (the DiT4DiT head): MEASURED_SKINNY.
+template <int MT, int NW, int KW, bool FOLD>
+__global__ __launch_bounds__(NW * 64) void skinny_staged_kernel(GemmArgs g) {
+  constexpr bool WD = MT == 4 && NW * KW == 1024;   // 80 rows x 2 KB would be the whole LDS
+  constexpr int MR = MT * 16, ROWS = MR + (WD ? 0 : 16);
+  __shared__ __attribute__((aligned(1024))) bf16 sm[NW][ROWS * KW];
+  __shared__ float2 s_st[FOLD ? NW : 1][MR];
+  __shared__ float s_piv[MR];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l16 = lane & 15, lg = lane >> 4;
+  const int M = (int)g.M, N = (int)g.N, K = (int)g.K;
+  const int n0 = blockIdx.x * 16, k0 = wave * KW;
+  const uint32_t lda2 = (uint32_t)g.lda * 2u, ldw2 = (uint32_t)g.ldw * 2u, kb = (uint32_t)k0 * 2u;
+  bf16* const my = &sm[wave][0];
+  bf16x8 wf[WD ? KW / 32 : 1];
+  if (k0 < K) {
+    const auto rw = buffer_rsrc(g.w + (int64_t)n0 * g.ldw, (uint32_t)min(16, N - n0) * ldw2);
+    if constexpr (WD) {
+#pragma unroll
+      for (int s = 0; s < KW / 32; ++s) wf[s] = buffer_load8(rw, (uint32_t)l16 * ldw2 + kb + (uint32_t)(4 * s + lg) * 16u);
+    } else {
+      panel_stage<KW, 16>(rw, ldw2, kb, my + MR * KW, lane);
+    }
+    panel_stage<KW, MR>(buffer_rsrc(g.a, (uint32_t)M * lda2), lda2, kb, my, lane);
+  }
+  // each thread's epilogue operands, and the rows' pivots, in flight with the panels
+  constexpr int EPT = (MR * 16 + NW * 64 - 1) / (NW * 64);
+  EpiIn ep[EPT];
+#pragma unroll
+  for (int u = 0; u < EPT; ++u) {
+    const int t = tid + u * NW * 64;
+    ep[u] = epilogue_load(g, std::min(t >> 4, M - 1), std::min(n0 + (t & 15), N - 1));
+  }
+  float piv[MT], s1[MT], s2[MT];
+  if constexpr (FOLD) {
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+      piv[i] = to_f(g.a[(int64_t)std::min(i * 16 + l16, M - 1) * g.lda]);
+      s1[i] = 0.f;
+      s2[i] = 0.f;
+    }
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  f32x4 acc[MT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  if (k0 < K) {
+    panel_wait();
+#pragma unroll
+    for (int s = 0; s < KW / 32; ++s) {
+      const bf16x8 w = WD ? wf[s] : panel_frag<KW>(my, MR, s, l16, lg);
+#pragma unroll
+      for (int i = 0; i < MT; ++i) {
+        const bf16x8 af = panel_frag<KW>(my, 16 * i, s, l16, lg);
+        acc[i] = mfma16(w, af, acc[i]);
+        if constexpr (FOLD) {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            const float d = to_f(af[e]) - piv[i];
+            s1[i] += d;
+            s2[i] += d * d;
+          }
+        }
+      }
+    }
+  }
+  if constexpr (FOLD) {
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+      s1[i] = group4_sum(s1[i]);
+      s2[i] = group4_sum(s2[i]);
+      if (lg == 0) {
+        s_st[wave][i * 16 + l16] = make_float2(s1[i], s2[i]);
+        if (wave == 0) s_piv[i * 16 + l16] = piv[i];
+      }
+    }
+  }
+  // the accumulators in the wave's own panel: lane (lg, l16) holds out[16 i + l16][n0 + 4 lg + e]
+  asm volatile("" ::: "memory");
+#pragma unroll
+  for (int i = 0; i < MT; ++i) *reinterpret_cast<f32x4*>(my + (i * 64 + lane) * 8) = acc[i];
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < EPT; ++u) {
+    const int t = tid + u * NW * 64, mr = t >> 4, c = t & 15, n = n0 + c;
+    if (t >= MR * 16 || mr >= M || n >= N) continue;
+    const int at = ((mr >> 4) * 64 + (c >> 2) * 16 + (mr & 15)) * 4 + (c & 3);
+    float p[NW], v = 0.f;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) p[w] = reinterpret_cast<const float*>(&sm[w][0])[at];
+#pragma unroll
+    for (int w = 0; w < NW; ++w) v += p[w];
+    if constexpr (FOLD) {
+      float t1 = 0.f, t2 = 0.f;
+#pragma unroll
+      for (int w = 0; w < NW; ++w) { t1 += s_st[w][mr].x; t2 += s_st[w][mr].y; }
+      const float invk = 1.0f / (float)K;
+      const float dm = t1 * invk;
+      const float rstd = rsqrtf(fmaxf(t2 * invk - dm * dm, 0.f) + g.eps);
+      v = rstd * (v - (s_piv[mr] + dm) * (g.csum ? ep[u].csum : 0.f));
+    }
+    epilogue_finish(g, mr, n, v, ep[u]);
+  }
+}
+
 // ---------------------------------------------------------------------------------------
 // partial_kernel: MT m-tiles (M <= 16*MT).  A workgroup owns 16 output columns over one K
 // slice of 4*32*STEPS; each of its 4 waves takes a quarter of the slice with every load
@@ -1378,11 +1486,40 @@ static void launch_skinny(const GemmArgs& a, int pro, hipStream_t s) {
   }
 }
 
+// Staged panels address a (M rows) and 16 weight rows with 32-bit byte offsets, and a wave's whole
+// KW-wide range has to lie inside K.
+static bool panel_ok(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldw, int kw) {
+  return K % kw == 0 && M * lda * 2 < (1LL << 31) && ldw < (1LL << 25) && N < (1LL << 31) - 16 && K < (1LL << 30);
+}
+
+// the staged form of a skinny product, where its panels cover K; false: not launched
+template <int MT>
+static bool launch_skinny_staged(const GemmArgs& a, int pro, hipStream_t s) {
+  const dim3 grid((unsigned)(round_up(a.N, 16) / 16));
+  auto ok = [&](int kw) { return panel_ok(a.M, a.N, a.K, a.lda, a.ldw, kw); };
+  if (pro == FAM_PRO_LN_FOLDED) {
+    if (a.K <= 512 && ok(64)) FAM_LAUNCH((skinny_staged_kernel<MT, 8, 64, true>), grid, dim3(512), 0, s, a);
+    else if (a.K > 512 && a.K <= 1024 && ok(128)) FAM_LAUNCH((skinny_staged_kernel<MT, 8, 128, true>), grid, dim3(512), 0, s, a);
+    else return false;
+    return true;
+  }
+  if (pro != FAM_PRO_NONE) return false;
+  if (a.K <= 256 && ok(64)) FAM_LAUNCH((skinny_staged_kernel<MT, 4, 64, false>), grid, dim3(256), 0, s, a);
+  else if (a.K > 256 && a.K <= 512 && ok(128)) FAM_LAUNCH((skinny_staged_kernel<MT, 4, 128, false>), grid, dim3(256), 0, s, a);
+  else if (a.K > 512 && a.K <= 1024 && ok(256)) FAM_LAUNCH((skinny_staged_kernel<MT, 4, 256, false>), grid, dim3(256), 0, s, a);
+  else if (MT == 1 && a.K > 1024 && a.K <= 2048 && ok(256)) {
+    // (16 rows of activations and 16 of weights x 4 KB: 128 KB)
+    if constexpr (MT == 1) FAM_LAUNCH((skinny_staged_kernel<1, 8, 256, false>), grid, dim3(512), 0, s, a);
+  } else return false;
+  return true;
+}
+
 // 8 waves with 4 k-steps each cover K <= 1024 in one chunk; longer K takes 16 waves with
 // 8 k-steps each (K <= 4096 in one chunk), more chunks beyond that.
 // The folded LayerNorm always takes 8 waves (its row sums need the registers).
 template <int MT>
 static void launch_skinny_k(const GemmArgs& a, int pro, hipStream_t s) {
+  if (launch_skinny_staged<MT>(a, pro, s)) return;
   if (a.K <= 1024 || pro == FAM_PRO_LN_FOLDED) launch_skinny<MT, 8, 4>(a, pro, s);
   else launch_skinny<MT, 16, 8>(a, pro, s);
 }
@@ -1754,12 +1891,6 @@ extern "C" int fam_gemm_partial_splits(int64_t M, int64_t N, int64_t K) {
   int st, sp;
   partial_plan(M, N, K, &st, &sp);
   return M > 128 && st >= 0 ? 0 : sp;
-}
-
-// Staged panels address a (M rows) and 16 weight rows with 32-bit byte offsets, and a wave's whole
-// KW-wide range has to lie inside K.
-static bool panel_ok(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldw, int kw) {
-  return K % kw == 0 && M * lda * 2 < (1LL << 31) && ldw < (1LL << 25) && N < (1LL << 31) - 16 && K < (1LL << 30);
 }
 
 template <int MT>
