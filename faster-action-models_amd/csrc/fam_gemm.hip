@@ -470,7 +470,8 @@ __global__ __launch_bounds__(NW * 64) void skinny_kernel(GemmArgs g) {
 // skinny_staged_kernel: the same product and epilogue (no prologue, or the folded LayerNorm) with
 // staged panels, NW waves of KW columns covering K (a multiple of KW).  The row sums of the folded
 // form come from the fragments the MFMAs use; it takes 8 waves, so that a SIMD's two waves share
-// them, the plain form 4.  17 rows x 768 (the DiT4DiT head): MEASURED_SKINNY.
+// them, the plain form 4.  The DiT4DiT head (17 rows, K = 768, about 50 such launches a step): 2100 ->
+// 1934 us for a call of 4 steps.
 template <int MT, int NW, int KW, bool FOLD>
 __global__ __launch_bounds__(NW * 64) void skinny_staged_kernel(GemmArgs g) {
   constexpr bool WD = MT == 4 && NW * KW == 1024;   // 80 rows x 2 KB would be the whole LDS
