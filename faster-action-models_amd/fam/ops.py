@@ -21,7 +21,7 @@ Tensors must be bf16 CUDA (HIP) tensors with a contiguous last dimension; anythi
 raises -- there is no fallback implementation.  Outputs are new tensors allocated on the
 input's device, launches go to torch's current stream.
 
-Each of these functions is a thin wrapper over a ``torch.library`` custom operator in the
+Each of these functions has a ``torch.library`` custom operator in the
 ``fam`` namespace (``torch.ops.fam.adaln``, ``rope``, ``attention``, ``linear``,
 ``euler_step``) with a fake implementation, so ``torch.compile(fullgraph=True)`` and
 ``torch.export`` trace through them as single graph nodes, the way the reference's own
@@ -41,16 +41,39 @@ from . import _capi
 from ._capi import call
 
 _BF16 = torch.bfloat16
+_PLAIN_TYPES = (torch.Tensor, torch.nn.Parameter)
 
 
 def _stream(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
+
+
+def _plain(*tensors) -> bool:
+    """True for an ordinary eager call: plain tensors (or None), nothing that records, traces or
+    transforms operators -- a compiler, a jit trace, a dispatch or function mode (fake and proxy
+    tensors, export), a functorch transform (vmap, grad, jvp), forward-mode duals, a gradient to
+    record, the profiler.  Then the operator would do nothing but call its implementation, and the
+    wrappers below call it themselves: the dispatcher's way through a Python operator costs a call
+    5 us (ops.linear at 32 rows 17.8 -> 8.5 us a call with the views and checks it no longer makes,
+    adaln_forward 20.4 -> 10.6 us; the kernels take 4 and 7 us)."""
+    if torch.compiler.is_compiling():
+        return False
+    grad = torch.is_grad_enabled()
+    for t in tensors:
+        if t is not None and (type(t) not in _PLAIN_TYPES or (grad and t.requires_grad)):
+            return False
+    return not (torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
+                or torch._C._functorch.peek_interpreter_stack() is not None
+                or torch.autograd.forward_ad._current_level >= 0 or torch._C._get_tracing_state() is not None
+                or torch._C._autograd._profiler_enabled())
 
 
 def _check(t: torch.Tensor, name: str, dtype=_BF16, device: bool = True) -> None:
     """dtype / last-dim checks, and (device=True) that t lives on a HIP device.  The fake
     implementations run the same checks with device=False, so a traced graph rejects what the
     real operator would."""
+    if type(t) in _PLAIN_TYPES and t.dtype is dtype and t.is_cuda and t.dim() > 0 and t.stride(-1) == 1:
+        return
     if not isinstance(t, torch.Tensor):
         raise TypeError(f"{name} must be a tensor")
     if device and t.device.type != "cuda":
@@ -62,7 +85,7 @@ def _check(t: torch.Tensor, name: str, dtype=_BF16, device: bool = True) -> None
 
 
 def _rows(x: torch.Tensor) -> Tuple[torch.Tensor, int, int, int]:
-    """View x as [B*S, D]; returns (2-D view, rows, rows_per_batch, D)."""
+    """x's rows: (x or a [B*S, D] view of it, rows, rows_per_batch, D)."""
     D = x.shape[-1]
     if x.dim() == 3:
         B, S = x.shape[0], x.shape[1]
@@ -70,6 +93,10 @@ def _rows(x: torch.Tensor) -> Tuple[torch.Tensor, int, int, int]:
         B, S = 1, x.shape[0]
     else:
         raise ValueError(f"expected a 2-D or 3-D tensor, got shape {tuple(x.shape)}")
+    if S > 1 and x.is_contiguous():
+        # the rows as they lie: callers read the address and the row pitch, stride(-2) (with S = 1
+        # that stride may be anything)
+        return x, B * S, S, D
     x2 = x.reshape(B * S, D)
     if x2.stride(-1) != 1:
         x2 = x2.contiguous()
@@ -80,6 +107,12 @@ def _rows(x: torch.Tensor) -> Tuple[torch.Tensor, int, int, int]:
 def _broadcast_mod(t: torch.Tensor, x: torch.Tensor, name: str) -> Tuple[torch.Tensor, int, int]:
     """Broadcast shift/scale to x's shape; returns (tensor, batch stride, row stride)."""
     _check(t, name)
+    if t.dim() == 3 and x.dim() == 3:
+        # [B or 1, S or 1, D] with aligned rows, read in place: the strides that expand would give
+        (tb, ts, td), (B, S, D) = t.shape, x.shape
+        bs, rs = t.stride(0) if tb == B else 0, t.stride(1) if ts == S else 0
+        if td == D and tb in (1, B) and ts in (1, S) and t.stride(2) == 1 and not (bs % 8 or rs % 8 or t.data_ptr() % 16):
+            return t, bs, rs
     tb = torch.broadcast_to(t, x.shape)
     if tb.stride(-1) != 1:
         tb = tb.contiguous()
@@ -96,7 +129,7 @@ def _broadcast_mod(t: torch.Tensor, x: torch.Tensor, name: str) -> Tuple[torch.T
 def _adaln_launch(x: torch.Tensor, shift, scale, weight, bias, eps: float) -> torch.Tensor:
     _check(x, "x")
     x2, rows, rpb, D = _rows(x)
-    y = torch.empty((rows, D), dtype=_BF16, device=x.device)
+    y = torch.empty(x.shape, dtype=_BF16, device=x.device)
     sh_p = sc_p = None
     bs = rs = 0
     if shift is not None:
@@ -115,19 +148,28 @@ def _adaln_launch(x: torch.Tensor, shift, scale, weight, bias, eps: float) -> to
     if bias is not None:
         _check(bias, "ln bias")
         bc = bias.contiguous()
-    call("fam_adaln", x2.data_ptr(), x2.stride(0), sh_p, sc_p, bs, rs,
+    call("fam_adaln", x2.data_ptr(), x2.stride(-2), sh_p, sc_p, bs, rs,
          wc.data_ptr() if wc is not None else None, bc.data_ptr() if bc is not None else None,
          y.data_ptr(), D, rows, rpb, D, float(eps), _stream(x))
-    return y.reshape(x.shape)
+    return y
+
+
+def _adaln_impl(x, shift, scale, weight, bias, eps: float) -> torch.Tensor:
+    if (shift is None) != (scale is None):
+        raise ValueError("adaln: shift and scale go together")
+    return _adaln_launch(x, shift, scale, weight, bias, eps)
+
+
+def _adaln(x, shift, scale, weight, bias, eps: float) -> torch.Tensor:
+    f = _adaln_impl if _plain(x, shift, scale, weight, bias) else torch.ops.fam.adaln
+    return f(x, shift, scale, weight, bias, eps)
 
 
 @torch.library.custom_op("fam::adaln", mutates_args=())
 def _adaln_op(x: torch.Tensor, shift: Optional[torch.Tensor], scale: Optional[torch.Tensor],
               weight: Optional[torch.Tensor], bias: Optional[torch.Tensor], eps: float) -> torch.Tensor:
     """LayerNorm over the last dim (optional affine), then optional modulation (1 + scale), + shift."""
-    if (shift is None) != (scale is None):
-        raise ValueError("adaln: shift and scale go together")
-    return _adaln_launch(x, shift, scale, weight, bias, eps)
+    return _adaln_impl(x, shift, scale, weight, bias, eps)
 
 
 @_adaln_op.register_fake
@@ -147,22 +189,22 @@ def adaln_forward(x: torch.Tensor, norm: torch.nn.LayerNorm, shift: torch.Tensor
     used); shift/scale broadcast as [B,1,D] (per sample) or [B,S,D] (per token)."""
     w = norm.weight if getattr(norm, "elementwise_affine", False) else None
     b = norm.bias if getattr(norm, "elementwise_affine", False) else None
-    return torch.ops.fam.adaln(x, shift, scale, w, b, float(norm.eps))
+    return _adaln(x, shift, scale, w, b, float(norm.eps))
 
 
 def layer_norm(x: torch.Tensor, weight: Optional[torch.Tensor], bias: Optional[torch.Tensor], eps: float) -> torch.Tensor:
     """nn.LayerNorm forward over the last dim (FB/wan_video_dit.py:258-261)."""
-    return torch.ops.fam.adaln(x, None, None, weight, bias, float(eps))
+    return _adaln(x, None, None, weight, bias, float(eps))
 
 
 def modulate_layer_norm(x: torch.Tensor, shift: torch.Tensor, scale: torch.Tensor, eps: float = 1e-6) -> torch.Tensor:
     """modulate(LayerNorm(x, affine=False), shift, scale) -- the CAE form (CA/wan_video_dit.py:590-591)."""
-    return torch.ops.fam.adaln(x, shift, scale, None, None, float(eps))
+    return _adaln(x, shift, scale, None, None, float(eps))
 
 
 def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
     """RMSNorm.forward: bf16(x*rsqrt(mean(x^2)+eps)) * weight (FB/wan_video_dit.py:156-167)."""
-    return torch.ops.fam.rope(x, None, 1, "none", weight, float(eps))
+    return _rope(x, None, 1, "none", weight, float(eps))
 
 
 class RMSNorm(torch.nn.Module):
@@ -220,8 +262,7 @@ def rope_tables(freqs: torch.Tensor, layout: str, device: torch.device):
         raise ValueError("layout 'complex' needs a complex freqs tensor")
     if layout != "complex" and freqs.is_complex():
         raise ValueError(f"layout {layout!r} needs a real freqs tensor")
-    key = (freqs.data_ptr(), tuple(freqs.shape), tuple(freqs.stride()), freqs.dtype, str(freqs.device),
-           freqs._version, layout, str(device))
+    key = (freqs.data_ptr(), freqs.shape, freqs.stride(), freqs.dtype, freqs.device, freqs._version, layout, device)
     hit = _TABLES.get(key)
     if hit is not None:
         _TABLES.move_to_end(key)
@@ -255,18 +296,18 @@ def _rope_launch(x: torch.Tensor, freqs: Optional[torch.Tensor], num_heads: int,
     if weight is not None:
         _check(weight, "weight")
     x2, rows, S, D = _rows(x)
-    y = torch.empty((rows, D), dtype=_BF16, device=x.device)
+    y = torch.empty(x.shape, dtype=_BF16, device=x.device)
     wc = weight.contiguous() if weight is not None else None
     w_p = wc.data_ptr() if wc is not None else None
     if layout == "none":
-        call("fam_rmsnorm_rope", x2.data_ptr(), x2.stride(0), y.data_ptr(), D, rows, 1, D, w_p, float(eps),
+        call("fam_rmsnorm_rope", x2.data_ptr(), x2.stride(-2), y.data_ptr(), D, rows, 1, D, w_p, float(eps),
              None, None, 0, 0, 0, _stream(x))
-        return y.reshape(x.shape)
+        return y
     _rope_shape(x, freqs, num_heads)
     cos, sin, trs, tes = rope_tables(freqs, layout, x.device)
-    call("fam_rmsnorm_rope", x2.data_ptr(), x2.stride(0), y.data_ptr(), D, rows, S, D, w_p, float(eps),
+    call("fam_rmsnorm_rope", x2.data_ptr(), x2.stride(-2), y.data_ptr(), D, rows, S, D, w_p, float(eps),
          cos.data_ptr(), sin.data_ptr(), trs, tes, D // num_heads, _stream(x))
-    return y.reshape(x.shape)
+    return y
 
 
 def _rope_shape(x: torch.Tensor, freqs: Optional[torch.Tensor], num_heads: int) -> None:
@@ -286,6 +327,10 @@ def _rope_op(x: torch.Tensor, freqs: Optional[torch.Tensor], num_heads: int, lay
              weight: Optional[torch.Tensor], eps: float) -> torch.Tensor:
     """Optional RMSNorm (weight given; bf16 rounding before the weight) then the rotation of
     `layout` ('complex', 'cat', 'interleaved', or 'none' for the norm alone)."""
+    return _rope_impl(x, freqs, num_heads, layout, weight, eps)
+
+
+def _rope_impl(x, freqs, num_heads: int, layout: str, weight, eps: float) -> torch.Tensor:
     if layout not in ("none", "complex", "cat", "interleaved"):
         raise ValueError(f"unknown RoPE layout {layout!r}")
     return _rope_launch(x, freqs, num_heads, layout, weight, eps)
@@ -303,11 +348,16 @@ def _rope_fake(x, freqs, num_heads, layout, weight, eps):
     return x.new_empty(x.shape)
 
 
+def _rope(x, freqs, num_heads: int, layout: str, weight, eps: float) -> torch.Tensor:
+    f = _rope_impl if _plain(x, freqs, weight) else torch.ops.fam.rope
+    return f(x, freqs, num_heads, layout, weight, eps)
+
+
 def rope_apply(x: torch.Tensor, freqs: torch.Tensor, num_heads: int) -> torch.Tensor:
     """Rotary embedding with the FB/FG call signature: freqs complex [S,1,Dh/2] or packed
     real cat(cos, sin) [S,1,Dh] (FB/wan_video_dit.py:58-70, FG/wan_video_dit.py:193-215).
     A real table in CA's interleaved packing is rejected (it belongs to rope_apply_cae)."""
-    return torch.ops.fam.rope(x, freqs, int(num_heads), "complex" if freqs.is_complex() else "cat", None, 0.0)
+    return _rope(x, freqs, int(num_heads), "complex" if freqs.is_complex() else "cat", None, 0.0)
 
 
 def rope_apply_cae(x: torch.Tensor, freqs: torch.Tensor, num_heads: int, force_complex: bool = False) -> torch.Tensor:
@@ -316,14 +366,14 @@ def rope_apply_cae(x: torch.Tensor, freqs: torch.Tensor, num_heads: int, force_c
     reference's arithmetic route; the rotation is the same.  A real table in FG's
     cat(cos, sin) packing is rejected (it belongs to rope_apply)."""
     del force_complex
-    return torch.ops.fam.rope(x, freqs, int(num_heads), "complex" if freqs.is_complex() else "interleaved", None,
+    return _rope(x, freqs, int(num_heads), "complex" if freqs.is_complex() else "interleaved", None,
                               0.0)
 
 
 def rms_norm_rope(x: torch.Tensor, weight: torch.Tensor, eps: float, freqs: torch.Tensor, num_heads: int,
                   layout: str = "complex") -> torch.Tensor:
     """rope_apply(RMSNorm(x), freqs) in one kernel (the q/k post-processing, FG/mot.py:786-816)."""
-    return torch.ops.fam.rope(x, freqs, int(num_heads), layout, weight, float(eps))
+    return _rope(x, freqs, int(num_heads), layout, weight, float(eps))
 
 
 # --------------------------------------------------------------------------- attention
@@ -434,6 +484,12 @@ def _attention_op(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, mask: Optio
     return _attention_launch(q, k, v, num_heads, mask, scale, k_prefix, v_prefix, None, num_splits, None)
 
 
+def _attention(q, k, v, mask, num_heads: int, scale, k_prefix, v_prefix, num_splits: int) -> torch.Tensor:
+    if _plain(q, k, v, mask, k_prefix, v_prefix):
+        return _attention_launch(q, k, v, num_heads, mask, scale, k_prefix, v_prefix, None, num_splits, None)
+    return torch.ops.fam.attention(q, k, v, mask, num_heads, scale, k_prefix, v_prefix, num_splits)
+
+
 @_attention_op.register_fake
 def _attention_fake(q, k, v, mask, num_heads, scale, k_prefix, v_prefix, num_splits):
     for t, n in ((q, "q"), (k, "k"), (v, "v")):
@@ -456,7 +512,7 @@ def attention_bshd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, num_heads:
     normalisation from fam_gemm_final sums of squares) the launch is direct, not an operator."""
     if out is not None or qk_norm is not None:
         return _attention_launch(q, k, v, num_heads, mask, scale, k_prefix, v_prefix, out, num_splits, qk_norm)
-    return torch.ops.fam.attention(q, k, v, mask, int(num_heads), scale, k_prefix, v_prefix, int(num_splits))
+    return _attention(q, k, v, mask, int(num_heads), scale, k_prefix, v_prefix, int(num_splits))
 
 
 def flash_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, num_heads: int,
@@ -466,28 +522,41 @@ def flash_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, num_heads
     if not compatibility_mode:
         raise NotImplementedError("Only compatibility mode is implemented for flash attention. "
                                   "Please set compatibility_mode=True.")
-    return torch.ops.fam.attention(q, k, v, ctx_mask, int(num_heads), None, None, None, 1)
+    return _attention(q, k, v, ctx_mask, int(num_heads), None, None, None, 1)
 
 
 # --------------------------------------------------------------------------- linear
 @torch.library.custom_op("fam::linear", mutates_args=())
 def _linear_op(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor]) -> torch.Tensor:
     """y = x W^T + b, bf16 in and out, fp32 accumulation."""
+    return _linear_impl(x, weight, bias)
+
+
+def _linear_impl(x, weight, bias) -> torch.Tensor:
     _check(x, "x")
     _check(weight, "weight")
     K = x.shape[-1]
     N = weight.shape[0]
     if weight.dim() != 2 or weight.shape[1] != K:
         raise ValueError(f"weight {tuple(weight.shape)} does not match input features {K}")
-    x2 = x.reshape(-1, K)
-    if x2.stride(-1) != 1:
-        x2 = x2.contiguous()
-    M = x2.shape[0]
     w = weight if weight.is_contiguous() else weight.contiguous()
     b = None
     if bias is not None:
         _check(bias, "bias")
         b = bias.contiguous()
+    if K % 8 == 0 and K > 0 and N > 0 and x.is_contiguous() and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0:
+        # rows and weight as they lie: no 2-D views are made
+        M = x.numel() // K
+        y = torch.empty((*x.shape[:-1], N), dtype=_BF16, device=x.device)
+        d = _capi.GemmDesc(x.data_ptr(), K, w.data_ptr(), K, b.data_ptr() if b is not None else None, y.data_ptr(), N,
+                           M, N, K)
+        d.rows_per_batch, d.gate_ns = max(M, 1), 1
+        call("fam_gemm", C.byref(d), _stream(x))
+        return y
+    x2 = x.reshape(-1, K)
+    if x2.stride(-1) != 1:
+        x2 = x2.contiguous()
+    M = x2.shape[0]
     y = torch.empty((M, N), dtype=_BF16, device=x.device)
     aligned = (K % 8 == 0 and x2.stride(0) % 8 == 0 and x2.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
     if not aligned:
@@ -514,7 +583,7 @@ def _linear_fake(x, weight, bias):
 
 def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
     """y = x W^T + b for bf16 x [..., K], W [N, K] (nn.Linear)."""
-    return torch.ops.fam.linear(x, weight, bias)
+    return (_linear_impl if _plain(x, weight, bias) else torch.ops.fam.linear)(x, weight, bias)
 
 
 def gemm(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], out: torch.Tensor, *,
@@ -532,24 +601,15 @@ def gemm(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], out: to
     if prologue == _capi.FAM_PRO_LN_FOLDED:
         if pro_w is None or pro_w.dtype != torch.float32 or pro_w.numel() != N or not pro_w.is_contiguous():
             raise ValueError("FAM_PRO_LN_FOLDED needs pro_w = fp32 contiguous [N] column sums of w")
-    d = _capi.GemmDesc()
-    d.a, d.lda = a.data_ptr(), a.stride(0)
-    d.w, d.ldw = w.data_ptr(), w.stride(0)
-    d.bias = bias.data_ptr() if bias is not None else None
-    d.out, d.ldo = out.data_ptr(), out.stride(0)
-    d.M, d.N, d.K = M, N, K
-    d.prologue = prologue
-    d.pro_w = pro_w.data_ptr() if pro_w is not None else None
-    d.pro_b = pro_b.data_ptr() if pro_b is not None else None
-    d.pro_shift = pro_shift.data_ptr() if pro_shift is not None else None
-    d.pro_scale = pro_scale.data_ptr() if pro_scale is not None else None
-    d.pro_mod_bs, d.pro_mod_rs, d.pro_eps = pro_mod_bs, pro_mod_rs, float(pro_eps)
-    d.act = act
-    d.res, d.ldr = (res.data_ptr(), res.stride(0)) if res is not None else (None, 0)
-    d.gate = gate.data_ptr() if gate is not None else None
-    d.gate_bs, d.gate_rs, d.gate_ns = gate_bs, gate_rs, gate_ns
-    d.rows_per_batch = rows_per_batch if rows_per_batch is not None else max(M, 1)
-    d.out_f32 = int(out_f32)
+    # one positional construction (field order of fam_gemm_desc): 27 attribute writes cost 2 us
+    d = _capi.GemmDesc(
+        a.data_ptr(), a.stride(0), w.data_ptr(), w.stride(0), bias.data_ptr() if bias is not None else None,
+        out.data_ptr(), out.stride(0), M, N, K, prologue, pro_w.data_ptr() if pro_w is not None else None,
+        pro_b.data_ptr() if pro_b is not None else None, pro_shift.data_ptr() if pro_shift is not None else None,
+        pro_scale.data_ptr() if pro_scale is not None else None, pro_mod_bs, pro_mod_rs, float(pro_eps), act,
+        res.data_ptr() if res is not None else None, res.stride(0) if res is not None else 0,
+        gate.data_ptr() if gate is not None else None, gate_bs, gate_rs, gate_ns,
+        rows_per_batch if rows_per_batch is not None else max(M, 1), int(out_f32))
     if ws is not None:
         if ws.dtype != torch.float32 or not ws.is_contiguous() or ws.device != a.device:
             raise ValueError("ws must be a contiguous fp32 tensor on the device of a")
@@ -728,7 +788,7 @@ def euler_step(model_output: torch.Tensor, delta: torch.Tensor, sample: torch.Te
         delta = torch.tensor(float(delta))
     if out is not None:
         return _euler_launch(model_output, delta, sample, out)
-    return torch.ops.fam.euler_step(model_output, delta, sample)
+    return (_euler_launch if _plain(model_output, delta, sample) else torch.ops.fam.euler_step)(model_output, delta, sample)
 
 
 class WanContinuousFlowMatchScheduler:

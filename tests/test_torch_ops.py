@@ -312,3 +312,34 @@ def test_rope_tables_accept_a_half_precision_table_in_the_right_packing(dtype):
         ops.rope_tables(inter, "cat", torch.device("cpu"))
     with pytest.raises(ValueError, match="rope_apply "):
         ops.rope_tables(cat, "interleaved", torch.device("cpu"))
+
+
+def test_plain_calls_are_only_the_ordinary_eager_ones():
+    """The wrappers call an operator's implementation themselves only where nothing watches operators:
+    every mode, transform or gradient that the dispatcher serves has to go through it."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+    from fam import ops
+    a, w = torch.zeros(2, 8), torch.nn.Parameter(torch.zeros(3, 8))
+    with torch.no_grad():
+        assert ops._plain(a, w, None)
+    assert not ops._plain(a, w)                       # a parameter with grad mode on
+    assert ops._plain(a, w.detach())
+    seen = []
+    torch.func.vmap(lambda t: (seen.append(ops._plain(t)), t)[1])(a)
+    torch.func.jvp(lambda t: (seen.append(ops._plain(t)), t)[1], (a,), (a,))
+    with torch.autograd.forward_ad.dual_level():
+        seen.append(ops._plain(torch.autograd.forward_ad.make_dual(a, a)))
+    with TorchDispatchMode():
+        seen.append(ops._plain(a))
+    with torch.device("meta"):                        # a function mode
+        seen.append(ops._plain(a))
+    with FakeTensorMode() as mode:
+        fake = mode.from_tensor(a)
+    seen.append(ops._plain(fake))
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]):
+        seen.append(ops._plain(a))
+    assert len(seen) == 7 and not any(seen), seen
+    got = []
+    torch.jit.trace(lambda t: (got.append(ops._plain(t)), t + 1)[1], a, check_trace=False)
+    assert got and not any(got)

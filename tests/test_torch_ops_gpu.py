@@ -579,3 +579,34 @@ def test_vfp8_row_ops(fw, D):
     rxo, rq, rs = O.vfp8_add_ln_mod_q8(x.float(), x2.float(), sh, sc, eps)
     assert xo.dtype == BF and torch.equal(xo.cpu().float(), rxo)
     cmp("add_ln_mod_q8", (q, s), (rq, rs))
+
+
+@pytest.mark.parametrize("B,S", [(1, 7), (3, 1), (1, 1), (2, 5)])
+def test_direct_calls_equal_the_operators(B, S):
+    """ops.* called plainly (no dispatcher, rows and modulation read in place) and torch.ops.fam.* give the
+    same bits, over inputs whose size-1 dimensions have strides of their own, transposed batches, column
+    windows and modulation rows in every broadcast form."""
+    from fam import ops
+    D, N = 1024, 520
+    g = torch.Generator().manual_seed(5)
+
+    def rn(*s):
+        return torch.randn(*s, generator=g).to(torch.bfloat16).cuda()
+    odd = torch.as_strided(rn(4 * B * S * D), (B, S, D), (S * D, D if S > 1 else 8 * 5, 1))
+    xs = [rn(B, S, D), rn(S, B, D).transpose(0, 1), rn(B, S, D + 64)[..., 32:32 + D], odd]
+    w, b, nw = rn(N, D), rn(N), rn(D)
+    mods = [rn(B, 1, 6 * D), rn(1, 1, 6 * D), rn(B, S, 6 * D), rn(1, S, 2 * D + 8), rn(2 * D)]
+    if B * S > 1:                                     # (one odd-pitched row is refused: no copy is made of it)
+        mods.append(rn(1, 1, 2 * D + 1))
+    ang = torch.rand(S, 1, 32, dtype=torch.float64, generator=g)
+    freqs = torch.polar(torch.ones_like(ang), ang)
+    for x in xs:
+        assert torch.equal(ops.linear(x, w, b), torch.ops.fam.linear(x, w, b))
+        assert torch.equal(ops.rms_norm(x, nw, 1e-6), torch.ops.fam.rope(x, None, 1, "none", nw, 1e-6))
+        assert torch.equal(ops.rms_norm_rope(x, nw, 1e-6, freqs, 16), torch.ops.fam.rope(x, freqs, 16, "complex", nw, 1e-6))
+        for m in mods:
+            sh, sc = m[..., :D], m[..., D:2 * D]
+            y = ops.modulate_layer_norm(x, sh, sc, 1e-6)
+            ref = torch.ops.fam.adaln(x, sh.expand(x.shape).contiguous(), sc.expand(x.shape).contiguous(), None, None, 1e-6)
+            assert torch.equal(y, ref) and y.is_contiguous() and y.shape == x.shape
+        assert torch.equal(ops.flash_attention(x, x, x, 16), torch.ops.fam.attention(x, x, x, None, 16, None, None, None, 1))
