@@ -61,6 +61,12 @@ struct GemmArgs {
   const float* csum;   // FAM_PRO_LN_FOLDED: sum_k w[n, k], fp32 [N]
 };
 
+// fam_conv3x3: the GEMM's a is an h x w image of channels-last rows, c channels; magic = ceil(2^32 / c).
+struct ConvArgs {
+  int h, w, c, stride;
+  uint32_t magic;
+};
+
 __device__ __forceinline__ float apply_act(float v, int act) {
   if (act == FAM_ACT_GELU_TANH) return gelu_tanh(v);
   if (act == FAM_ACT_SILU) return silu(v);
@@ -1204,8 +1210,19 @@ __device__ __forceinline__ void mfma_acc(f32x4& acc, const bf16x8& w, const bf16
 // blocks): 8 waves in two K groups of 4; group g takes the K blocks g, g + 2, ... into its own
 // two slots, so each SIMD runs two waves although the grid leaves one workgroup per CU; group 1
 // then parks its accumulators in LDS for group 0 to add (in a fixed order) before the epilogue.
-template <int WFM, int WFN, int KG = 1, int NS = 2>
-__global__ __launch_bounds__(256 * KG) void big_kernel(GemmArgs g, int tiles_m, int tiles_n, int vec8, int ksplit, int raw) {
+// CONV (fam_conv3x3): the rows of A are the 3 x 3 neighbourhoods of an image's pixels, never laid
+// out in memory: column k is channel k % C of tap k / C, so a lane's 16-byte chunk (C % 8 == 0)
+// is one pixel's.  Per row a lane keeps the byte offset of its window's corner and a mask of the
+// taps inside the image, and a tap outside reads past the descriptor's range, which stores zeros.
+// CONV = 2 (C % 64 == 0): a K block lies in one tap, found on the scalar unit.  CONV = 1: each
+// lane derives its own tap and channel (one multiply-high).
+// Measured with bias (im2col + GEMM -> this): 112 x 224 pixels, 160 -> 160 channels 41.3 -> 21.4
+// us; 56 x 112, 320 -> 320 34.2 -> 20.1; 28 x 56, 640 -> 640 33.8 -> 27.7 (29.2 with CONV = 1);
+// 256 x 256, 320 -> 512 294 -> 161 us (1.2 PFLOP/s).  Against the GEMM alone on rows laid out
+// before, the 64 x 64 tiles lose 10-20 % to the address arithmetic, the larger ones nothing.
+template <int WFM, int WFN, int KG = 1, int NS = 2, int CONV = 0>
+__global__ __launch_bounds__(256 * KG) void big_kernel(GemmArgs g, int tiles_m, int tiles_n, int vec8, int ksplit, int raw,
+                                                         ConvArgs cv) {
   // the A part of a slot holds BMA >= BM rows, a multiple of 64 (a 224-row tile also loads the
   // next 32 rows, unused: measured 2-4 % faster than 7 loads per wave per block)
   constexpr int BM = 32 * WFM, BN = 32 * WFN, BK = 64, BMA = (BM + 63) / 64 * 64;
@@ -1247,7 +1264,8 @@ __global__ __launch_bounds__(256 * KG) void big_kernel(GemmArgs g, int tiles_m, 
 
   const int Mi = (int)g.M, Ni = (int)g.N;
   const uint32_t lda2 = (uint32_t)g.lda * 2u, ldw2 = (uint32_t)g.ldw * 2u;
-  const auto ra = buffer_rsrc(g.a + (int64_t)m0 * g.lda, (uint32_t)(Mi - m0) * lda2);
+  const auto ra = CONV ? buffer_rsrc(g.a, (uint32_t)(cv.h * cv.w) * lda2)
+                       : buffer_rsrc(g.a + (int64_t)m0 * g.lda, (uint32_t)(Mi - m0) * lda2);
   const auto rw = buffer_rsrc(g.w + (int64_t)n0 * g.ldw, (uint32_t)(Ni - n0 < BN ? Ni - n0 : BN) * ldw2);
   const int lr = lane >> 3;
   const uint32_t lc16 = (uint32_t)(((lane & 7) ^ lr) * 16);
@@ -1255,6 +1273,23 @@ __global__ __launch_bounds__(256 * KG) void big_kernel(GemmArgs g, int tiles_m, 
   const int nball = (int)(g.K / BK);
   const int kb0 = (int)((int64_t)split * nball / ksplit), nbs = (int)((int64_t)(split + 1) * nball / ksplit) - kb0;
   const int nb = nbs / KG;   // blocks of this K group (KG = 2 runs with an even count only)
+  uint32_t cbase[CONV ? NIA : 1], ctaps[CONV ? NIA : 1];
+  if constexpr (CONV) {
+    const int wo = cv.stride == 1 ? cv.w : cv.w >> 1, pad = cv.stride == 1 ? 1 : 0;
+#pragma unroll
+    for (int p = 0; p < NIA; ++p) {
+      const int m = m0 + 8 * (wave + 4 * p) + lr;
+      const int oy = m / wo, y = cv.stride * oy - pad, x = cv.stride * (m - oy * wo) - pad;
+      uint32_t xm = 0, t = 0;
+#pragma unroll
+      for (int k = 0; k < 3; ++k) xm |= (uint32_t)((uint32_t)(x + k) < (uint32_t)cv.w) << k;
+#pragma unroll
+      for (int k = 0; k < 3; ++k) t |= (uint32_t)(y + k) < (uint32_t)cv.h ? xm << (3 * k) : 0u;
+      ctaps[p] = m < Mi ? t : 0u;
+      // modulo 2^32: exact once a tap inside is added
+      cbase[p] = (uint32_t)(y * cv.w + x) * lda2 + (CONV == 2 ? lc16 : 0u);
+    }
+  }
   // load p of this wave for the group's block blk (of this split) into slot: A rows 8 (wave + 4p)
   // .. + 7 for p < NIA, else W rows 8 (wave + 4 (p - NIA)) .. + 7; blocks past the end re-read
   // the last one (unused).  The group's block j is block KG j + kgi of the split.
@@ -1263,8 +1298,15 @@ __global__ __launch_bounds__(256 * KG) void big_kernel(GemmArgs g, int tiles_m, 
     const uint32_t kb = (uint32_t)(kb0 + KG * (blk < nb ? blk : nb - 1) + kgi) * (BK * 2);
     if (p < NIA) {
       const int r = wave + 4 * p;
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, FAM_LDS(smg + slot * SS + r * 512), 16,
-                                               voa + (uint32_t)(8 * r) * lda2 + kb, 0, 0, 0);
+      if constexpr (CONV) {
+        const uint32_t col2 = CONV == 2 ? kb : kb + lc16, tap = __umulhi(col2 >> 1, cv.magic), kh = tap * 11u >> 5;   // tap / 3, tap < 16
+        const uint32_t in = cbase[p] + (kh * (uint32_t)cv.w + (tap - 3u * kh)) * lda2 + (col2 - tap * (uint32_t)cv.c * 2u);
+        const uint32_t vo = ctaps[p] >> tap & 1u ? in : 0x7ffffff0u;
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, FAM_LDS(smg + slot * SS + r * 512), 16, vo, 0, 0, 0);
+      } else {
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, FAM_LDS(smg + slot * SS + r * 512), 16,
+                                                 voa + (uint32_t)(8 * r) * lda2 + kb, 0, 0, 0);
+      }
     } else {
       const int r = wave + 4 * (p - NIA);
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, FAM_LDS(smg + slot * SS + SA + r * 512), 16,
@@ -1538,8 +1580,8 @@ static bool big_ok(const fam_gemm_desc* d) {
 }
 
 // raw: fp32 planes without epilogue (always with ksplit > 1)
-template <int WFM, int WFN, int KG = 1>
-static void launch_big(const GemmArgs& a, hipStream_t s, int ksplit = 1, bool raw = false) {
+template <int WFM, int WFN, int KG = 1, int CONV = 0>
+static void launch_big(const GemmArgs& a, hipStream_t s, int ksplit = 1, bool raw = false, const ConvArgs& cv = ConvArgs{}) {
   const int tm = (int)((a.M + 32 * WFM - 1) / (32 * WFM)), tn = (int)((a.N + 32 * WFN - 1) / (32 * WFN));
   const unsigned grid = (unsigned)(((tm * tn * ksplit + 7) / 8) * 8);
   // 8-column epilogue vectors when every 8-column group of the operands is 16-byte aligned
@@ -1548,12 +1590,12 @@ static void launch_big(const GemmArgs& a, hipStream_t s, int ksplit = 1, bool ra
                    (!a.gate || (a.gbs % 8 == 0 && a.grs % 8 == 0 && al16(a.gate)));
   if constexpr (WFM == 2 && WFN == 2 && KG == 1) {
     if ((int64_t)tm * tn * ksplit <= 2 * (int64_t)fam_host::device_cus()) {
-      FAM_LAUNCH((big_kernel<2, 2, 1, 4>), dim3(grid), dim3(256), 0, s, a, tm, tn, vec8, ksplit, (int)(raw || ksplit > 1));
+      FAM_LAUNCH((big_kernel<2, 2, 1, 4, CONV>), dim3(grid), dim3(256), 0, s, a, tm, tn, vec8, ksplit, (int)(raw || ksplit > 1), cv);
       return;
     }
   }
-  FAM_LAUNCH((big_kernel<WFM, WFN, KG>), dim3(grid), dim3(256 * KG), 0, s, a, tm, tn, vec8, ksplit,
-             (int)(raw || ksplit > 1));
+  FAM_LAUNCH((big_kernel<WFM, WFN, KG, 2, CONV>), dim3(grid), dim3(256 * KG), 0, s, a, tm, tn, vec8, ksplit,
+             (int)(raw || ksplit > 1), cv);
 }
 
 // Tile of the big kernel: the candidate with the least estimated time on the busiest CU,
@@ -1659,6 +1701,22 @@ static void big_plan_split(int64_t M, int64_t N, int64_t K, int64_t ws_floats, b
     }
 }
 
+// One launch of the big kernel, no split.
+template <int CONV>
+static void launch_big_unsplit(const GemmArgs& a, hipStream_t s, const ConvArgs& cv = ConvArgs{}) {
+  int fm = 8, fn = 8;
+  big_plan(a.M, a.N, a.act, &fm, &fn, true);
+  if (fm == 8) launch_big<8, 8, 1, CONV>(a, s, 1, false, cv);
+  else if (fm == 7) launch_big<7, 8, 1, CONV>(a, s, 1, false, cv);
+  else if (fm == 4 && fn == 3) launch_big<4, 3, 1, CONV>(a, s, 1, false, cv);
+  else if (fm == 4 && !big_prefers_64(a.M, a.N, a.K)) {
+    // at most one 128 x 128 workgroup per CU: two K groups per workgroup (an even block count)
+    const int64_t tiles = ((a.M + 127) / 128) * ((a.N + 127) / 128);
+    if (tiles <= fam_host::device_cus() && (a.K / 64) % 2 == 0) launch_big<4, 4, 2, CONV>(a, s, 1, false, cv);
+    else launch_big<4, 4, 1, CONV>(a, s, 1, false, cv);
+  } else launch_big<2, 2, 1, CONV>(a, s, 1, false, cv);
+}
+
 template <int BM, int BN, int WM>
 static void launch_tiled(const GemmArgs& a, int pro, hipStream_t s) {
   dim3 grid((unsigned)(round_up(a.N, BN) / BN), (unsigned)(round_up(a.M, BM) / BM));
@@ -1685,6 +1743,25 @@ static bool stream_single(const fam_gemm_desc* d) {
   int steps, splits, nwv = 8;
   partial_plan(d->M, d->N, d->K, &steps, &splits, &nwv);
   return steps < 0 && splits == 1 && nwv == 8;
+}
+
+// The descriptor as kernel arguments.
+static GemmArgs gemm_args(const fam_gemm_desc* d) {
+  GemmArgs a{};
+  a.a = (const bf16*)d->a; a.lda = d->lda;
+  a.w = (const bf16*)d->w; a.ldw = d->ldw;
+  a.bias = (const bf16*)d->bias;
+  a.out = (bf16*)d->out; a.ldo = d->ldo;
+  a.M = d->M; a.N = d->N; a.K = d->K;
+  a.pw = (const bf16*)d->pro_w; a.pb = (const bf16*)d->pro_b;
+  a.shift = (const bf16*)d->pro_shift; a.scale = (const bf16*)d->pro_scale;
+  a.mbs = d->pro_mod_bs; a.mrs = d->pro_mod_rs; a.eps = d->pro_eps;
+  a.act = d->act;
+  a.res = (const bf16*)d->res; a.ldr = d->ldr;
+  a.gate = (const bf16*)d->gate; a.gbs = d->gate_bs; a.grs = d->gate_rs; a.gns = d->gate_ns;
+  a.rpb = d->rows_per_batch;
+  a.out_f32 = d->out_f32 != 0;
+  return a;
 }
 
 extern "C" int fam_gemm(const fam_gemm_desc* d, void* stream) {
@@ -1722,20 +1799,7 @@ extern "C" int fam_gemm(const fam_gemm_desc* d, void* stream) {
   FAM_REQUIRE(d->N <= (int64_t)65535 * 16 && d->M <= (int64_t)65535 * 64, FAM_ERR_UNSUPPORTED, "fam_gemm: too large");
   if (d->M == 0) return FAM_OK;
 
-  GemmArgs a{};
-  a.a = (const bf16*)d->a; a.lda = d->lda;
-  a.w = (const bf16*)d->w; a.ldw = d->ldw;
-  a.bias = (const bf16*)d->bias;
-  a.out = (bf16*)d->out; a.ldo = d->ldo;
-  a.M = d->M; a.N = d->N; a.K = d->K;
-  a.pw = (const bf16*)d->pro_w; a.pb = (const bf16*)d->pro_b;
-  a.shift = (const bf16*)d->pro_shift; a.scale = (const bf16*)d->pro_scale;
-  a.mbs = d->pro_mod_bs; a.mrs = d->pro_mod_rs; a.eps = d->pro_eps;
-  a.act = d->act;
-  a.res = (const bf16*)d->res; a.ldr = d->ldr;
-  a.gate = (const bf16*)d->gate; a.gbs = d->gate_bs; a.grs = d->gate_rs; a.gns = d->gate_ns;
-  a.rpb = d->rows_per_batch;
-  a.out_f32 = d->out_f32 != 0;
+  GemmArgs a = gemm_args(d);
   if (d->prologue == FAM_PRO_LN_FOLDED) {
     a.csum = (const float*)d->pro_w;
     a.pw = nullptr;
@@ -1763,22 +1827,38 @@ extern "C" int fam_gemm(const fam_gemm_desc* d, void* stream) {
   else if (skinny && d->M <= 32) launch_skinny_k<2>(a, d->prologue, s);
   else if (skinny) launch_skinny_k<4>(a, d->prologue, s);
   else if (big_ok(d)) {
-    int fm = 8, fn = 8;
-    big_plan(d->M, d->N, d->act, &fm, &fn, true);
-    if (fm == 8) launch_big<8, 8>(a, s);
-    else if (fm == 7) launch_big<7, 8>(a, s);
-    else if (fm == 4 && fn == 3) launch_big<4, 3>(a, s);
-    else if (fm == 4 && !big_prefers_64(d->M, d->N, d->K)) {
-      // at most one 128 x 128 workgroup per CU: two K groups per workgroup (an even block count)
-      const int64_t tiles = ((d->M + 127) / 128) * ((d->N + 127) / 128);
-      if (tiles <= fam_host::device_cus() && (d->K / 64) % 2 == 0) launch_big<4, 4, 2>(a, s);
-      else launch_big<4, 4>(a, s);
-    } else launch_big<2, 2>(a, s);
+    launch_big_unsplit<0>(a, s);
   } else if (round_up(d->M, 128) / 128 * (round_up(d->N, 128) / 128) >= 200) launch_tiled<128, 128, 2>(a, d->prologue, s);
   else launch_tiled<64, 64, 2>(a, d->prologue, s);
   return fam_host::check_launch("fam_gemm");
 }
 
+
+// The product in ks fp32 planes in ws, then their sum with d's epilogue.
+template <int CONV>
+static int launch_big_split(GemmArgs a, const fam_gemm_desc* d, int fm, int ks, float* ws, void* stream, const char* who,
+                            const ConvArgs& cv = ConvArgs{}) {
+  a.out = (bf16*)ws; a.ldo = d->N; a.out_f32 = 1;
+  a.bias = nullptr; a.res = nullptr; a.gate = nullptr; a.act = FAM_ACT_NONE; a.rpb = d->M;
+  hipStream_t s = (hipStream_t)stream;
+  if (fm == 8) launch_big<8, 8, 1, CONV>(a, s, ks, false, cv);
+  else if (fm == 7) launch_big<7, 8, 1, CONV>(a, s, ks, false, cv);
+  else if (fm == 4) launch_big<4, 4, 1, CONV>(a, s, ks, false, cv);
+  else launch_big<2, 2, 1, CONV>(a, s, ks, false, cv);
+  const int rc = fam_host::check_launch(who);
+  if (rc != FAM_OK) return rc;
+  fam_rowop_desc r{};
+  r.src = FAM_ROWSRC_PARTIALS;
+  r.partials = ws; r.splits = ks; r.split_stride = d->M * d->N; r.ldp = d->N;
+  r.M = d->M; r.N = d->N;
+  r.bias = d->bias; r.act = d->act;
+  r.res = d->res; r.ldr = d->ldr;
+  r.gate = d->gate; r.gate_bs = d->gate_bs; r.gate_rs = d->gate_rs; r.gate_ns = d->gate_ns;
+  r.rows_per_batch = d->rows_per_batch;
+  r.out = d->out; r.ldo = d->ldo; r.out_f32 = d->out_f32;
+  r.norm = FAM_ROWNORM_NONE;
+  return fam_rowop(&r, stream);
+}
 
 // fam_gemm with a workspace: products inside the big kernel's envelope may split K over
 // workgroups (big_plan_split), the fp32 planes summed in split order by fam_rowop, which also
@@ -1803,26 +1883,43 @@ extern "C" int fam_gemm_ws(const fam_gemm_desc* d, float* ws, int64_t ws_floats,
   GemmArgs a{};
   a.a = (const bf16*)d->a; a.lda = d->lda;
   a.w = (const bf16*)d->w; a.ldw = d->ldw;
-  a.out = (bf16*)ws; a.ldo = d->N; a.out_f32 = 1;
-  a.M = d->M; a.N = d->N; a.K = d->K; a.rpb = d->M;
-  hipStream_t s = (hipStream_t)stream;
-  if (fm == 8) launch_big<8, 8>(a, s, ks);
-  else if (fm == 7) launch_big<7, 8>(a, s, ks);
-  else if (fm == 4) launch_big<4, 4>(a, s, ks);
-  else launch_big<2, 2>(a, s, ks);
-  const int rc = fam_host::check_launch("fam_gemm_ws");
-  if (rc != FAM_OK) return rc;
-  fam_rowop_desc r{};
-  r.src = FAM_ROWSRC_PARTIALS;
-  r.partials = ws; r.splits = ks; r.split_stride = d->M * d->N; r.ldp = d->N;
-  r.M = d->M; r.N = d->N;
-  r.bias = d->bias; r.act = d->act;
-  r.res = d->res; r.ldr = d->ldr;
-  r.gate = d->gate; r.gate_bs = d->gate_bs; r.gate_rs = d->gate_rs; r.gate_ns = d->gate_ns;
-  r.rows_per_batch = d->rows_per_batch;
-  r.out = d->out; r.ldo = d->ldo; r.out_f32 = d->out_f32;
-  r.norm = FAM_ROWNORM_NONE;
-  return fam_rowop(&r, stream);
+  a.M = d->M; a.N = d->N; a.K = d->K;
+  return launch_big_split<0>(a, d, fm, ks, ws, stream, "fam_gemm_ws");
+}
+
+// The neighbourhoods of an image's pixels times w^T on the big kernel, with fam_gemm_ws's plans
+// and epilogue; the product with the neighbourhoods laid out in memory reads the same operands in
+// the same order and gives the same bits.  Laying them out (fam_im2col3x3) writes 9 C columns a
+// pixel only for the product to read them back: a fifth of the 224 x 448 VAE encode.
+extern "C" int fam_conv3x3(const fam_gemm_desc* d, int64_t H, int64_t W, int64_t C, int64_t stride, float* ws,
+                           int64_t ws_floats, void* stream) {
+  FAM_REQUIRE(d && d->a && d->w && d->out, FAM_ERR_INVALID_ARG, "fam_conv3x3: null pointer");
+  FAM_REQUIRE(ws_floats >= 0 && (ws_floats == 0 || (ws && ((uintptr_t)ws & 15u) == 0)), FAM_ERR_INVALID_ARG,
+              "fam_conv3x3: workspace must be 16-byte aligned");
+  FAM_REQUIRE((stride == 1 || (stride == 2 && H % 2 == 0 && W % 2 == 0)) && H >= 1 && W >= 1 && H < (1 << 24) &&
+                  W < (1 << 24) && d->M == (H / stride) * (W / stride),
+              FAM_ERR_INVALID_ARG, "fam_conv3x3: stride 1, or 2 with even H and W; M = output pixels");
+  FAM_REQUIRE(C >= 8 && C % 8 == 0 && C <= 16384 && d->K % 64 == 0 && d->K >= 9 * C && d->K < 9 * C + 64 &&
+                  d->lda >= C && d->lda % 8 == 0 && d->ldw >= d->K && d->ldw % 8 == 0 && d->N >= 1 && d->ldo >= d->N,
+              FAM_ERR_INVALID_ARG, "fam_conv3x3: C % 8 == 0, K = 9 C rounded up to 64, lda >= C, ldw >= K, ldo >= N");
+  FAM_REQUIRE(fam_host::aligned16(d->a) && fam_host::aligned16(d->w), FAM_ERR_INVALID_ARG,
+              "fam_conv3x3: a and w must be 16-byte aligned");
+  FAM_REQUIRE(d->act >= FAM_ACT_NONE && d->act <= FAM_ACT_GELU_ERF && d->rows_per_batch >= 1 && (!d->gate || d->res),
+              FAM_ERR_INVALID_ARG, "fam_conv3x3: act, rows_per_batch or gate");
+  FAM_REQUIRE(big_ok(d) && H * W * d->lda * 2 < ((int64_t)1 << 31) - 16, FAM_ERR_UNSUPPORTED,
+              "fam_conv3x3: at least 128 output pixels, N %% 4 == 0, 4-element aligned vectors, below 2 GiB, no prologue");
+  const GemmArgs a = gemm_args(d);
+  const ConvArgs cv{(int)H, (int)W, (int)C, (int)stride,
+                    (uint32_t)(((((uint64_t)1) << 32) + (uint64_t)C - 1) / (uint64_t)C)};   // exact for columns < 2^32 / C
+  int fm = 8, fn = 8, ks = 1;
+  if (ws_floats >= 2 * d->M * d->N) big_plan_split(d->M, d->N, d->K, ws_floats, false, &fm, &fn, &ks);
+  const bool one_tap = C % 64 == 0;   // every K block of 64 within one tap
+  if (ks > 1)
+    return one_tap ? launch_big_split<2>(a, d, fm, ks, ws, stream, "fam_conv3x3", cv)
+                   : launch_big_split<1>(a, d, fm, ks, ws, stream, "fam_conv3x3", cv);
+  if (one_tap) launch_big_unsplit<2>(a, (hipStream_t)stream, cv);
+  else launch_big_unsplit<1>(a, (hipStream_t)stream, cv);
+  return fam_host::check_launch("fam_conv3x3");
 }
 
 

@@ -1,8 +1,8 @@
 // The Wan2.2 VAE encoder's first frame (the policy call's prologue) around the library's GEMM.
 // Activations are channels-last rows, one row per pixel ([h*w, C] bf16), so a 1x1 convolution
-// is a GEMM over the rows and a 3x3 one is a GEMM over an im2col operand whose row is the
-// pixel's 3x3 neighbourhood, taps outermost ((kh*3 + kw)*C + c), zero-padded to a multiple of
-// 64 columns.  The kernels here are the non-GEMM steps, each one elementwise pass over the bytes
+// is a GEMM over the rows and a 3x3 one a GEMM over the pixels' 3x3 neighbourhoods, taps
+// outermost ((kh*3 + kw)*C + c), zero-padded to a multiple of 64 columns: fam_conv3x3 gathers
+// them itself, and below its 128 output pixels im2col3x3_kernel lays them out.  The kernels here are the non-GEMM steps, each one elementwise pass over the bytes
 // it moves (the middle attention's softmax is one wave per row).
 #include "fam_common.h"
 

@@ -8,9 +8,9 @@ it is a 2-D convolution with its last temporal tap, and the downsample3d time_co
 for a second chunk, :162-167) does not run.
 
 Layout: activations are channels-last rows, one per pixel ([h*w, C] bf16).  A 1x1 convolution
-is one GEMM over the rows; a 3x3 convolution is fam_im2col3x3 (the pixel's neighbourhood, taps
-outermost, zero-padded to a multiple of 64 columns) followed by a GEMM with the weight laid out
-the same way; biases, the residual adds and the Down_ResidualBlock shortcut are GEMM epilogues.
+is one GEMM over the rows; a 3x3 convolution is a GEMM over the pixels' neighbourhoods (taps
+outermost, zero-padded to a multiple of 64 columns), which fam_conv3x3 gathers while it multiplies
+and, below its 128 output pixels, fam_im2col3x3 lays out first; biases, the residual adds and the Down_ResidualBlock shortcut are GEMM epilogues.
 The GEMMs go through fam_gemm_ws with one shared fp32 workspace, so the deep levels (392 to
 1568 pixels, K up to 5760) split K over workgroups instead of leaving most CUs idle.  The middle AttentionBlock (one head, C = 640 wide, h*w tokens) is two fam_gemm
 products around fam_softmax_rows: S = q k^T, P = softmax(S / sqrt(C)), O = P v0 + b_v, where
@@ -180,11 +180,10 @@ class FusedWanVAEEncoder:
                           (x_copy.data_ptr(), x_copy.stride(0), h, w, ci, co, 2 if t_down else 1, 2, None, 0,
                            avg.data_ptr(), co), "avgdown", 2 * (x_copy.numel() + avg.numel()))
                 self.stages[f"l{i}.avg"] = avg
-                a = self._im2col(f"l{i}.down", x, h, w, co, 2)
                 wr, br = conv3(f"{pre}{cfg.num_res_blocks}.resample.1.weight", f"{pre}{cfg.num_res_blocks}.resample.1.bias")
+                xn = z2((h // 2) * (w // 2), co)
+                self._conv(f"l{i}.down", x, h, w, co, 2, wr, br, xn, res=avg)
                 h, w = h // 2, w // 2
-                xn = z2(h * w, co)
-                self._gemm(f"l{i}.down", a, wr, br, xn, res=avg)
                 x = xn
             self.stages[f"level{i}"] = x
 
@@ -195,10 +194,9 @@ class FusedWanVAEEncoder:
         t = z2(h * w, c)
         self._add("head.norm", "fam_chan_rmsnorm", (x.data_ptr(), c, h * w, c, self._k(gamma("encoder.head.0.gamma")),
                                                      _capi.FAM_ACT_SILU, t.data_ptr(), c), "norm", 4 * x.numel())
-        a = self._im2col("head", t, h, w, c, 1)
         wh, bh = conv3("encoder.head.2.weight", "encoder.head.2.bias")
         hz = z2(h * w, 2 * z)
-        self._gemm("head", a, wh, bh, hz)
+        self._conv("head", t, h, w, c, 1, wh, bh, hz)
         self.stages["head"] = hz
         wmu, bmu = conv1x1("conv1.weight", "conv1.bias", rows=slice(0, z))
         mu = z2(h * w, z)
@@ -237,7 +235,7 @@ class FusedWanVAEEncoder:
         self.meta.append({"name": name, "kernel": kind, "bytes": int(nbytes)})
 
     def _gemm(self, name, a, w, bias, out, *, M=None, K=None, lda=None, ldw=None, ldo=None, res=None,
-              out_f32=False):
+              out_f32=False, conv=None):
         self._keep += [a, w, out] + ([bias] if bias is not None else []) + ([res] if res is not None else [])
         d = _capi.GemmDesc()
         d.a, d.lda = a.data_ptr(), lda if lda is not None else a.stride(0)
@@ -252,14 +250,25 @@ class FusedWanVAEEncoder:
         d.rows_per_batch = max(d.M, 1)
         d.out_f32 = int(out_f32)
         self._descs.append(d)
-        f, lib = self.lib.fam_gemm_ws, self.lib
+        fname = "fam_gemm_ws" if conv is None else "fam_conv3x3"
+        f, lib, grid = getattr(self.lib, fname), self.lib, conv or ()
 
         def run(stream):
-            rc = f(C.byref(d), *self._ws_args, stream)
+            rc = f(C.byref(d), *grid, *self._ws_args, stream)
             if rc != 0:
-                raise _capi.FamError(f"fam_gemm_ws[{name}]", rc, lib.fam_last_error().decode(errors="replace"))
+                raise _capi.FamError(f"{fname}[{name}]", rc, lib.fam_last_error().decode(errors="replace"))
         self.steps.append(run)
-        self.meta.append({"name": name, "kernel": "gemm", "bytes": 2 * (d.M * d.K + d.N * d.K + d.M * d.N)})
+        self.meta.append({"name": name, "kernel": "gemm", "bytes": 2 * (a.numel() + d.N * d.K + d.M * d.N) if conv
+                          else 2 * (d.M * d.K + d.N * d.K + d.M * d.N)})
+
+    def _conv(self, name, x, h, w, c, stride, wt, bias, out, *, res=None):
+        """A 3x3 convolution of the h x w rows x: fam_conv3x3 inside its limits (same
+        plan and bits), else the neighbourhoods laid out and a GEMM."""
+        if (out.shape[0] >= 128 and wt.shape[0] % 4 == 0 and c <= 16384 and h * w * x.stride(0) < 1 << 29
+                and wt.numel() < 1 << 29):
+            self._gemm(name, x, wt, bias, out, M=out.shape[0], res=res, conv=(h, w, c, stride))
+        else:
+            self._gemm(name, self._im2col(name, x, h, w, c, stride), wt, bias, out, res=res)
 
     def _im2col(self, name, x, h, w, c, stride):
         ho, wo = (h, w) if stride == 1 else (h // 2, w // 2)
@@ -291,18 +300,16 @@ class FusedWanVAEEncoder:
         t = z2(n, ci)
         self._add(pre + "norm0", "fam_chan_rmsnorm", (x.data_ptr(), x.stride(0), n, ci, self._k(gamma(pre + "residual.0.gamma")),
                                                       _capi.FAM_ACT_SILU, t.data_ptr(), ci), "norm", 4 * t.numel())
-        a = self._im2col(pre + "conv2", t, h, w, ci, 1)
         w2, b2 = conv3(pre + "residual.2.weight", pre + "residual.2.bias")
         y = z2(n, co)
-        self._gemm(pre + "conv2", a, w2, b2, y)
+        self._conv(pre + "conv2", t, h, w, ci, 1, w2, b2, y)
         self.stages[pre + "conv2"] = y
         t2 = z2(n, co)
         self._add(pre + "norm3", "fam_chan_rmsnorm", (y.data_ptr(), co, n, co, self._k(gamma(pre + "residual.3.gamma")),
                                                       _capi.FAM_ACT_SILU, t2.data_ptr(), co), "norm", 4 * t2.numel())
-        a2 = self._im2col(pre + "conv6", t2, h, w, co, 1)
         w6, b6 = conv3(pre + "residual.6.weight", pre + "residual.6.bias")
         out = z2(n, co)
-        self._gemm(pre + "conv6", a2, w6, b6, out, res=hs)
+        self._conv(pre + "conv6", t2, h, w, co, 1, w6, b6, out, res=hs)
         self.stages[pre + "out"] = out
         return out
 

@@ -502,6 +502,17 @@ int fam_gather_rows(const void* src, int64_t ld_src, int64_t src_rows, const int
 int fam_vae_patch_im2col(const void* img, int64_t H, int64_t W, void* out, int64_t ldo, void* stream);
 
 /*
+ * fam_conv3x3 -- fam_gemm_ws of the rows fam_im2col3x3 would write, without writing them: d->a is
+ * the H x W channels-last image x (d->lda = ldx), d->w the weight [N, K] with taps outermost and
+ * columns 9*C..K-1 zero, K = 9*C rounded up to 64, M the output pixels (stride 1 or 2 as
+ * fam_im2col3x3); bias, activation, gate, residual and output as fam_gemm, ws as fam_gemm_ws.
+ * Limits: C % 8 == 0, C <= 16384; no prologue; M >= 128, N % 4 == 0, H*W*ldx below 1 Gi elements
+ *         and 4-column aligned epilogue vectors (FAM_ERR_UNSUPPORTED otherwise).
+ */
+int fam_conv3x3(const fam_gemm_desc* d, int64_t H, int64_t W, int64_t C, int64_t stride, float* ws,
+                int64_t ws_floats, void* stream);
+
+/*
  * fam_im2col3x3 -- out[p, (kh*3 + kw)*C + c] = x[y, x', c] around output pixel p of the H x W
  * channels-last grid x (row stride ldx); stride 1: 'same' zero padding (CausalConv3d's spatial
  * padding); stride 2: zero padding at the bottom / right only and (H/2) x (W/2) outputs

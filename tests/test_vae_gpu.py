@@ -46,6 +46,51 @@ def test_im2col3x3(H, W, C, stride):
     assert torch.equal(got[:, 9 * C:], torch.zeros_like(got[:, 9 * C:]))
 
 
+# Edges of the image on every side of a tile, C below, off and above the 64-wide K block, both
+# strides, padded rows, and image sizes that reach each tile of the product and its split planes.
+@pytest.mark.parametrize("H,W,C,N,stride,ldx", [
+    (9, 17, 8, 12, 1, 8), (1, 130, 24, 64, 1, 32), (130, 1, 64, 20, 1, 64), (28, 56, 40, 100, 2, 48),
+    (16, 20, 160, 96, 1, 160), (14, 28, 640, 640, 1, 640), (56, 112, 320, 640, 2, 320), (96, 96, 80, 256, 1, 80),
+    (112, 224, 160, 160, 1, 160), (224, 256, 16, 512, 1, 16), (100, 125, 32, 1024, 1, 32), (128, 128, 56, 128, 1, 56)])
+def test_conv3x3_equals_im2col_gemm(H, W, C, N, stride, ldx):
+    """The same plan reads the same operands in the same order: the bits are the same."""
+    from fam import _capi
+    import ctypes
+    lib = _lib()
+    g = torch.Generator().manual_seed(H * 131 + W)
+    x = torch.full((H * W, ldx), float("nan"), dtype=BF)   # the padding columns are never used
+    x[:, :C] = torch.randn(H * W, C, generator=g).to(BF)
+    kp = (9 * C + 63) // 64 * 64
+    P = (H // stride) * (W // stride)
+    w = torch.zeros(N, kp, dtype=BF)
+    w[:, :9 * C] = (torch.randn(N, 9 * C, generator=g) / math.sqrt(9 * C)).to(BF)
+    x, w = x.cuda(), w.cuda()
+    bias, res = (torch.randn(*s, generator=g).to(BF).cuda() for s in ((N,), (P, N)))
+    rows = torch.empty(P, kp, dtype=BF, device="cuda")
+    assert lib.fam_im2col3x3(x.data_ptr(), ldx, H, W, C, stride, rows.data_ptr(), kp, kp, _s()) == 0
+    wsf = lib.fam_gemm_ws_floats(P, N, kp)
+    ws = torch.empty(max(wsf, 4), device="cuda")
+    outs = []
+    for conv in (False, True):
+        y = torch.empty(P, N, dtype=BF, device="cuda")
+        a = x if conv else rows
+        d = _capi.GemmDesc()
+        d.a, d.lda, d.w, d.ldw, d.bias = a.data_ptr(), a.stride(0), w.data_ptr(), kp, bias.data_ptr()
+        d.out, d.ldo, d.M, d.N, d.K, d.act = y.data_ptr(), N, P, N, kp, _capi.FAM_ACT_NONE
+        d.res, d.ldr, d.rows_per_batch = res.data_ptr(), N, P
+        if conv:
+            assert lib.fam_conv3x3(ctypes.byref(d), H, W, C, stride, ws.data_ptr(), wsf, _s()) == 0
+        else:
+            assert lib.fam_gemm_ws(ctypes.byref(d), ws.data_ptr(), wsf, _s()) == 0
+        outs.append(y)
+    assert torch.equal(outs[0], outs[1])
+    img = x[:, :C].float().t().reshape(1, C, H, W).cpu()
+    k = w[:, :9 * C].float().reshape(N, 3, 3, C).permute(0, 3, 1, 2).cpu()
+    img = F.pad(img, (1, 1, 1, 1)) if stride == 1 else F.pad(img, (0, 1, 0, 1))
+    ref = F.conv2d(img, k, bias.float().cpu(), stride=stride).reshape(N, P).t() + res.float().cpu()
+    assert _rel(outs[1], ref) <= 1e-2
+
+
 def test_vae_patch_im2col():
     H, W = 12, 20
     img = torch.randn(1, 3, H, W, generator=torch.Generator().manual_seed(2)).to(BF)
