@@ -139,6 +139,60 @@ def test_vae_avgdown(Cin, Cout, ft, fs):
         assert _rel(out, ref) <= 1e-2
 
 
+@pytest.mark.parametrize("rows", [1, 7, 33])
+@pytest.mark.parametrize("C", [8, 120, 128, 136, 160, 256, 264, 512, 520, 1024, 1032])
+def test_chan_rmsnorm_lane_groups(rows, C):
+    """Every lane group and both register forms, at the widths where they change; a row of zeros."""
+    from fam import _capi
+    g = torch.Generator().manual_seed(rows * 7 + C)
+    x = torch.randn(rows, C + 8, generator=g).to(BF)
+    x[rows // 2] = 0
+    gamma = (1 + 0.2 * torch.randn(C, generator=g)).to(BF)
+    y = torch.full((rows + 1, C + 16), 7.0, dtype=BF, device="cuda")
+    xd, gd = x.cuda(), gamma.cuda()
+    assert _lib().fam_chan_rmsnorm(xd.data_ptr(), C + 8, rows, C, gd.data_ptr(), _capi.FAM_ACT_SILU, y.data_ptr(),
+                                   C + 16, _s()) == 0
+    ref = F.silu(F.normalize(x[:, :C].double(), dim=1) * math.sqrt(C) * gamma.double())
+    # one bf16 rounding of a value whose fp32 error is far smaller
+    assert ((y[:rows, :C].cpu().double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 1e-6).all()
+    assert (y[rows] == 7).all() and (y[:, C:] == 7).all()
+
+
+@pytest.mark.parametrize("Cin,Cout,ft,fs,pad", [
+    (8, 8, 1, 1, 0), (8, 16, 2, 1, 8), (160, 160, 1, 2, 0), (24, 48, 2, 2, 8),   # 8 outputs a thread
+    (16, 16, 1, 2, 1), (12, 12, 1, 2, 0), (16, 8, 1, 2, 0), (16, 32, 1, 2, 0)])   # one output a thread
+def test_vae_avgdown_forms(Cin, Cout, ft, fs, pad):
+    """Both forms against exact group means of the folded layout, rows padded by `pad`."""
+    H, W = 10, 6
+    P = (H // fs) * (W // fs)
+    g = torch.Generator().manual_seed(Cin + Cout)
+    x, add = torch.randn(H * W, Cin + pad, generator=g).to(BF), torch.randn(P, Cout + pad, generator=g).to(BF)
+    xd, ad = x.cuda(), add.cuda()
+    ref = O.vae_avg_down(x[:, :Cin].double().t().reshape(1, Cin, H, W), Cout, ft, fs).reshape(Cout, -1).t()
+    for a in (None, ad):
+        out = torch.full((P + 1, Cout + pad), 7.0, dtype=BF, device="cuda")
+        assert _lib().fam_vae_avgdown(xd.data_ptr(), Cin + pad, H, W, Cin, Cout, ft, fs,
+                                      a.data_ptr() if a is not None else None, Cout + pad, out.data_ptr(), Cout + pad,
+                                      _s()) == 0
+        want = ref if a is None else ref + add[:, :Cout].double()
+        # one bf16 rounding; the fp32 sums of at most 8 values of magnitude < 8 are exact to 2^-18
+        assert ((out[:P, :Cout].cpu().double() - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -18).all()
+        assert (out[P] == 7).all() and (out[:, Cout:] == 7).all()
+
+
+@pytest.mark.parametrize("ldo", [128, 131])
+def test_vae_patch_im2col_rows(ldo):
+    H, W = 10, 14
+    img = torch.randn(3, H, W, generator=torch.Generator().manual_seed(5)).to(BF)
+    imgd = img.cuda()
+    out = torch.full((35, ldo), 7.0, dtype=BF, device="cuda")
+    assert _lib().fam_vae_patch_im2col(imgd.data_ptr(), H, W, out.data_ptr(), ldo, _s()) == 0
+    t = img.float().reshape(3, H // 2, 2, W // 2, 2).permute(0, 4, 2, 1, 3).reshape(1, 12, H // 2, W // 2)
+    ref = F.unfold(t, 3, padding=1).reshape(12, 9, 35).permute(2, 1, 0).reshape(35, 108)
+    assert torch.equal(out[:, :108].float().cpu(), ref)
+    assert (out[:, 108:128] == 0).all() and (out[:, 128:] == 7).all()
+
+
 def test_softmax_rows_and_affine():
     g = torch.Generator().manual_seed(5)
     s = torch.randn(9, 70, generator=g) * 4
