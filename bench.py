@@ -139,10 +139,10 @@ def measured_traffic(cls: str):
 
 
 # library kernel name (rocprofv3's Kernel_Name, "fam::<name>...") -> bench.py's kernel class
-_KERNEL_CLASSES = [("final_kernel", "gemm_final"), ("partial", "gemm_partial"), ("rowop", "rowop"),
+_KERNEL_CLASSES = [("final_", "gemm_final"), ("partial", "gemm_partial"), ("rowop", "rowop"),
                    ("attn_combine", "attn_combine"), ("attn_", "attention"), ("rmsnorm_rope", "rmsnorm_rope"),
                    ("add_mod", "modulation"), ("sinusoid", "sinusoid"), ("big_kernel", "gemm"),
-                   ("skinny_kernel", "gemm"), ("tiled_kernel", "gemm"), ("euler", "euler"), ("adaln", "adaln")]
+                   ("skinny_", "gemm"), ("tiled_kernel", "gemm"), ("euler", "euler"), ("adaln", "adaln")]
 
 
 def _kernel_class(name: str):
