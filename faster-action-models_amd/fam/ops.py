@@ -49,7 +49,8 @@ def _stream(t: torch.Tensor) -> int:
 
 
 def _plain(*tensors) -> bool:
-    """True for an ordinary eager call: plain tensors (or None), nothing that records, traces or
+    """True for an ordinary eager call: plain tensors (or None) whose memory holds their values (the
+    dispatcher resolves lazily conjugated, negated and zero tensors), nothing that records, traces or
     transforms operators -- a compiler, a jit trace, a dispatch or function mode (fake and proxy
     tensors, export), a functorch transform (vmap, grad, jvp), forward-mode duals, a gradient to
     record, the profiler.  Then the operator would do nothing but call its implementation, and the
@@ -60,7 +61,8 @@ def _plain(*tensors) -> bool:
         return False
     grad = torch.is_grad_enabled()
     for t in tensors:
-        if t is not None and (type(t) not in _PLAIN_TYPES or (grad and t.requires_grad)):
+        if t is not None and (type(t) not in _PLAIN_TYPES or (grad and t.requires_grad) or t.is_conj() or t.is_neg()
+                              or t._is_zerotensor()):
             return False
     return not (torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
                 or torch._C._functorch.peek_interpreter_stack() is not None
@@ -262,12 +264,15 @@ def rope_tables(freqs: torch.Tensor, layout: str, device: torch.device):
         raise ValueError("layout 'complex' needs a complex freqs tensor")
     if layout != "complex" and freqs.is_complex():
         raise ValueError(f"layout {layout!r} needs a real freqs tensor")
-    key = (freqs.data_ptr(), freqs.shape, freqs.stride(), freqs.dtype, freqs.device, freqs._version, layout, device)
+    # (a lazily conjugated or negated view has the address and version of its base)
+    key = (freqs.data_ptr(), freqs.shape, freqs.stride(), freqs.dtype, freqs.device, freqs._version, layout, device,
+           freqs.is_conj(), freqs.is_neg())
     hit = _TABLES.get(key)
     if hit is not None:
         _TABLES.move_to_end(key)
         return hit[1:]
-    S = freqs.shape[0]
+    S, source = freqs.shape[0], freqs
+    freqs = freqs.resolve_conj().resolve_neg()
     if layout == "complex":
         f = freqs.reshape(S, -1)
         cos = f.real.to(device=device, dtype=torch.float32).contiguous()
@@ -284,7 +289,7 @@ def rope_tables(freqs: torch.Tensor, layout: str, device: torch.device):
             res = (f, f[:, half:], f.stride(0), 1)
         else:
             res = (f, f[:, 1:], f.stride(0), 2)
-    _TABLES[key] = (freqs,) + res
+    _TABLES[key] = (source,) + res
     while len(_TABLES) > _TABLES_MAX:
         _TABLES.popitem(last=False)
     return res

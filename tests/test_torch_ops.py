@@ -343,3 +343,33 @@ def test_plain_calls_are_only_the_ordinary_eager_ones():
     got = []
     torch.jit.trace(lambda t: (got.append(ops._plain(t)), t + 1)[1], a, check_trace=False)
     assert got and not any(got)
+
+
+def test_plain_calls_exclude_lazily_stored_tensors():
+    """A conjugated, negated or zero tensor's memory does not hold its values: the dispatcher resolves it
+    before the implementation reads addresses, so such a call is not a plain one."""
+    z, r = torch.zeros(4, dtype=torch.complex64), torch.zeros(4)
+    assert ops._plain(z, r)
+    for t in (z.conj(), torch._neg_view(r), z.conj().imag, torch._efficientzerotensor((4,))):
+        assert not ops._plain(t) and not ops._plain(r, None, t)
+
+
+@pytest.mark.parametrize("first", ["table", "conjugate"])
+def test_rope_tables_of_a_conjugated_table_are_its_own(first):
+    """freqs.conj() is a view with the address, strides and version of freqs: each has tables of its own,
+    whichever is used first, and neither is served the other's.  So for a negated real table."""
+    dev = torch.device("cpu")
+    ang = torch.rand(8, 1, 16, dtype=torch.float64, generator=torch.Generator().manual_seed(11)) + 0.1
+    for dtype in (torch.complex128, torch.complex64):
+        f = torch.polar(torch.ones_like(ang), ang).to(dtype)
+        order = (f, f.conj()) if first == "table" else (f.conj(), f)
+        for t in order + order:                        # the second pass is served from the cache
+            cos, sin, _, _ = ops.rope_tables(t, "complex", dev)
+            sign = -1.0 if t.is_conj() else 1.0
+            assert not sin.is_neg() and torch.equal(cos, ang[:, 0].cos().to(f.real.dtype).float())
+            assert torch.allclose(sin, sign * ang[:, 0].sin().float(), rtol=1e-6)
+    t = _cat_table(8, 16)
+    order = (t, torch._neg_view(t)) if first == "table" else (torch._neg_view(t), t)
+    for v in order + order:
+        cos, sin, _, _ = ops.rope_tables(v, "cat", dev)
+        assert not cos.is_neg() and torch.equal(cos[:, :8], v.reshape(8, 16)[:, :8].clone())

@@ -610,3 +610,27 @@ def test_direct_calls_equal_the_operators(B, S):
             ref = torch.ops.fam.adaln(x, sh.expand(x.shape).contiguous(), sc.expand(x.shape).contiguous(), None, None, 1e-6)
             assert torch.equal(y, ref) and y.is_contiguous() and y.shape == x.shape
         assert torch.equal(ops.flash_attention(x, x, x, 16), torch.ops.fam.attention(x, x, x, None, 16, None, None, None, 1))
+
+
+@pytest.mark.parametrize("first", ["table", "conjugate"])
+def test_rope_apply_conjugated_table(first):
+    """rope_apply(x, freqs.conj()) rotates back, whichever of the table and its conjugate is used first;
+    lazily negated rows, weights and modulation are read as their values."""
+    from fam import ops
+    g = torch.Generator().manual_seed(12)
+    S, H, Dh = 9, 4, 64
+    x = _rand(g, 2, S, H * Dh)
+    ang = torch.rand(S, 1, Dh // 2, dtype=torch.float64, generator=g)
+    f = torch.polar(torch.ones_like(ang), ang)
+    xd, fd = x.cuda(), f.cuda()
+    for _ in range(2):
+        for t in ((fd, fd.conj()) if first == "table" else (fd.conj(), fd)):
+            ref = O.rope_apply(x.float(), f.conj() if t.is_conj() else f, H)
+            assert _rel(ops.rope_apply(xd, t, H), ref) <= 2e-2
+            assert torch.equal(ops.rope_apply(xd, t, H), ops.rope_apply(xd, t.resolve_conj(), H))
+    neg = torch._neg_view(xd)
+    w = _rand(g, 96, H * Dh).cuda()
+    assert torch.equal(ops.linear(neg, w), ops.linear(-xd, w))
+    assert torch.equal(ops.rope_apply(neg, fd, H), ops.rope_apply(-xd, fd, H))
+    assert torch.equal(ops.modulate_layer_norm(xd, neg, neg), ops.modulate_layer_norm(xd, -xd, -xd))
+    assert torch.equal(ops.flash_attention(neg, xd, neg, H), ops.flash_attention(-xd, xd, -xd, H))
