@@ -1176,8 +1176,11 @@ __global__ __launch_bounds__(256) void attn_cross_kernel(AttnArgs a) {
 // half-tile reads 32 contiguous bytes of row q (keys 32 hh .. + 31 of the tile, any alignment) and
 // trades every other dword with lane l ^ 32, so a tile costs a lane two 16-byte loads; they are in
 // flight under the softmax and P V of the tile before.  A wave none of whose 32 x 64 entries is set
-// leaves the tile's products out, one with all of them set skips the selects.  1592 x 1592 joint
-// mask, 24 x 128 heads: 273 us on attn_tiled_kernel, 60.5 us here.
+// leaves the tile's products out, one with all of them set skips the selects.  The softmax is as
+// exact as attn_tiled_kernel's, which these masks ran on before: an exact running max and a sum of
+// the rounded probabilities, with the first tile in halves.  1592 x 1592 joint mask, 24 x 128
+// heads: 273 us there, 64 here (61 with the lazy max below); error against float64 2.218e-3 there,
+// 2.217e-3 here, 2.334e-3 with the lazy max (peaked scores, x 5: 1.71, 1.69 and 1.94e-3).
 // KW = 2 (head dim 128, a grid of at most one workgroup per CU): 8 waves in two key groups of
 // 4; group g takes the tiles g, g + 2, g + 4, ... of the same 128 queries with its own LDS slots,
 // so each SIMD runs two waves (one's softmax under the other's MFMAs) although the grid leaves
@@ -1370,6 +1373,20 @@ __global__ __launch_bounds__(256 * KW, 2 / KW) void attn_long_kernel(AttnArgs a,
     else p = (const lds_bf16*)&Ks[buf][0][0] + koff_l + kt * 32 * KLD + ks * 16;
     return *reinterpret_cast<const __attribute__((address_space(3))) bf16x8*>(p);
   };
+  // the sum of a lane's 16 rounded probabilities of a half-tile, two per dot product with (1, 1)
+  auto sum_bf16 = [](const bf16x8 (&p)[2]) {
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    const bf16x2 one = {(__bf16)1.0f, (__bf16)1.0f};
+    float s[2] = {0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < 8; j += 2)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const bf16x2 v = {p[i][j], p[i][j + 1]};
+        s[i] = __builtin_amdgcn_fdot2_f32_bf16(v, one, s[i], false);
+      }
+    return s[0] + s[1];
+  };
   f32x16 acc[DT];
 #pragma unroll
   for (int d = 0; d < DT; ++d) acc[d] = f32x16{};
@@ -1382,8 +1399,8 @@ __global__ __launch_bounds__(256 * KW, 2 / KW) void attn_long_kernel(AttnArgs a,
   // without a key mask) sets the scores of keys past Sk to -inf, so full tiles carry no
   // per-score masking.  The group's next tile (t + KW) goes to the other buffer first, which the
   // last barrier released (zeros past Sk).
-  auto compute = [&](int t, auto tail_tag, auto buf_tag) {
-    constexpr bool TAIL = decltype(tail_tag)::value;
+  auto compute = [&](int t, auto tail_tag, auto buf_tag, auto split_tag) {
+    constexpr bool TAIL = decltype(tail_tag)::value, SPLIT = decltype(split_tag)::value;
     constexpr int buf = decltype(buf_tag)::value;
     bool some = false;
     if constexpr (QMASK) {
@@ -1440,43 +1457,62 @@ __global__ __launch_bounds__(256 * KW, 2 / KW) void attn_long_kernel(AttnArgs a,
     // online softmax (log2 domain).  The running max only moves when a score exceeds it by
     // more than 2^8 (or on the first tile), so the accumulator rescale is skipped on most
     // tiles; p <= 2^8 in between is exact in fp32 and bf16 keeps its relative precision.
-    float mraw = -INFINITY;
+    // QMASK: the max is exact and the sum is that of the rounded p, so that a query's largest
+    // probability so far is exactly 1 and the others' rounding errors meet in numerator and
+    // denominator (the sum costs two probabilities an instruction).
+    auto keys = [&](auto kt0_tag, auto kt1_tag) {   // half-tiles kt0 .. kt1 - 1
+      constexpr int kt0 = decltype(kt0_tag)::value, kt1 = decltype(kt1_tag)::value;
+      float mraw = -INFINITY;
 #pragma unroll
-    for (int kt = 0; kt < 2; ++kt)
+      for (int kt = kt0; kt < kt1; ++kt)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) mraw = fmaxf(mraw, st[kt][r]);
-    mraw = max_xor32(mraw);
-    const float mloc = mraw * sl2;   // sl2 > 0
-    if (__any(mloc > m_run + 8.0f)) {
-      const float m_new = fmaxf(m_run, mloc);
-      // max unchanged: 1; -inf: 0 (a query of its own mask rows may still have no key: -inf - -inf)
-      const float alpha = __builtin_amdgcn_exp2f(m_run - (QMASK && m_new == -INFINITY ? 0.f : m_new));
-      l_run *= alpha;
+        for (int r = 0; r < 16; ++r) mraw = fmaxf(mraw, st[kt][r]);
+      mraw = max_xor32(mraw);
+      const float mloc = mraw * sl2;   // sl2 > 0
+      if (__any(mloc > m_run + (QMASK ? 0.0f : 8.0f))) {
+        const float m_new = fmaxf(m_run, mloc);
+        // max unchanged: 1; -inf: 0 (a query of its own mask rows may still have no key: -inf - -inf)
+        const float alpha = __builtin_amdgcn_exp2f(m_run - (QMASK && m_new == -INFINITY ? 0.f : m_new));
+        l_run *= alpha;
 #pragma unroll
-      for (int d = 0; d < DT; ++d) acc[d] *= alpha;
-      m_run = m_new;
-    }
-    // (a query whose keys so far are all masked keeps m_run = -inf: its p are exp2(-inf) = 0)
-    const float m_use = MK && m_run == -INFINITY ? 0.f : m_run;
-    float psum = 0.f;
-    bf16x8 pf[2][2];
-#pragma unroll
-    for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const float pv = __builtin_amdgcn_exp2f(__builtin_fmaf(st[kt][r], sl2, -m_use));
-        psum += pv;
-        pf[kt][r / 8][r % 8] = to_bf(pv);
+        for (int d = 0; d < DT; ++d) acc[d] *= alpha;
+        m_run = m_new;
       }
-    psum = sum_xor32(psum);
-    l_run += psum;
-    // O^T += V^T P^T: k-step c of half kt covers keys kt*32 + 16c + {4hh..4hh+3, 8+4hh..8+4hh+3}
+      // (a query whose keys so far are all masked keeps m_run = -inf: its p are exp2(-inf) = 0)
+      const float m_use = MK && m_run == -INFINITY ? 0.f : m_run;
+      float psum = 0.f;
+      bf16x8 pf[2][2];
 #pragma unroll
-    for (int kt = 0; kt < 2; ++kt)
+      for (int kt = kt0; kt < kt1; ++kt)
 #pragma unroll
-      for (int c = 0; c < 2; ++c)
+        for (int r = 0; r < 16; ++r) {
+          const float pv = __builtin_amdgcn_exp2f(__builtin_fmaf(st[kt][r], sl2, -m_use));
+          if constexpr (!QMASK) psum += pv;
+          pf[kt][r / 8][r % 8] = to_bf(pv);
+        }
+      if constexpr (QMASK) {
 #pragma unroll
-        for (int d = 0; d < DT; ++d) acc[d] = mfma32(vfrag(buf, kt * 32 + 16 * c, d), pf[kt][c], acc[d]);
+        for (int kt = kt0; kt < kt1; ++kt) psum += sum_bf16(pf[kt]);
+      }
+      psum = sum_xor32(psum);
+      l_run += psum;
+      // O^T += V^T P^T: k-step c of half kt covers keys kt*32 + 16c + {4hh..4hh+3, 8+4hh..8+4hh+3}
+#pragma unroll
+      for (int kt = kt0; kt < kt1; ++kt)
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+#pragma unroll
+          for (int d = 0; d < DT; ++d) acc[d] = mfma32(vfrag(buf, kt * 32 + 16 * c, d), pf[kt][c], acc[d]);
+    };
+    using I0 = std::integral_constant<int, 0>;
+    using I1 = std::integral_constant<int, 1>;
+    using I2 = std::integral_constant<int, 2>;
+    if constexpr (SPLIT) {
+      keys(I0{}, I1{});
+      keys(I1{}, I2{});
+    } else {
+      keys(I0{}, I2{});
+    }
   };
   auto prefetch = [&](int t, int buf) {
     dma_kv(t, buf);
@@ -1490,10 +1526,10 @@ __global__ __launch_bounds__(256 * KW, 2 / KW) void attn_long_kernel(AttnArgs a,
     if constexpr (DMA) __builtin_amdgcn_s_waitcnt(0x0070);   // vmcnt(0) lgkmcnt(0): the next tile landed
     __syncthreads();
   };
-  auto tile = [&](int t, auto tail_tag, auto buf_tag) {
+  auto tile = [&](int t, auto tail_tag, auto buf_tag, auto split_tag) {
     constexpr int buf = decltype(buf_tag)::value;
     prefetch(t + 1, buf ^ 1);
-    compute(t, tail_tag, buf_tag);
+    compute(t, tail_tag, buf_tag, split_tag);
     finish(buf ^ 1);
   };
   // KW = 2: stage s holds tile 2 s + kg of each key group; a group whose tile is past the end
@@ -1502,8 +1538,8 @@ __global__ __launch_bounds__(256 * KW, 2 / KW) void attn_long_kernel(AttnArgs a,
     constexpr int buf = decltype(buf_tag)::value;
     const int tg = KW * s + kg;
     prefetch(tg + KW, buf ^ 1);
-    if (tg < nfull_kw) compute(tg, std::false_type{}, buf_tag);
-    else if (tg < ntiles_kw) compute(tg, std::true_type{}, buf_tag);
+    if (tg < nfull_kw) compute(tg, std::false_type{}, buf_tag, std::false_type{});
+    else if (tg < ntiles_kw) compute(tg, std::true_type{}, buf_tag, std::false_type{});
     finish(buf ^ 1);
   };
 
@@ -1516,17 +1552,27 @@ __global__ __launch_bounds__(256 * KW, 2 / KW) void attn_long_kernel(AttnArgs a,
   using T = std::true_type;
   using B0 = std::integral_constant<int, 0>;
   using B1 = std::integral_constant<int, 1>;
-  if constexpr (KW == 1) {
+  if constexpr (KW == 1 && QMASK) {
+    // the first tile in halves: with its max already exact after 32 keys the result is as near
+    // to the exact softmax as blocks of 32 keys throughout leave it (attn_tiled_kernel)
+    tile(0, F{}, B0{}, T{});
+    int t = 1;
+    for (; t + 1 < ntiles; t += 2) {
+      tile(t, F{}, B1{}, F{});
+      tile(t + 1, F{}, B0{}, F{});
+    }
+    if (t < ntiles) tile(t, F{}, B1{}, F{});
+  } else if constexpr (KW == 1) {
     int t = 0;
     for (; t + 1 < nfull; t += 2) {
-      tile(t, F{}, B0{});
-      tile(t + 1, F{}, B1{});
+      tile(t, F{}, B0{}, F{});
+      tile(t + 1, F{}, B1{}, F{});
     }
     if (t < nfull) {
-      tile(t, F{}, B0{});
-      if (t + 1 < ntiles) tile(t + 1, T{}, B1{});
+      tile(t, F{}, B0{}, F{});
+      if (t + 1 < ntiles) tile(t + 1, T{}, B1{}, F{});
     } else if (t < ntiles) {
-      tile(t, T{}, B0{});
+      tile(t, T{}, B0{}, F{});
     }
   } else {
     const int nst = (ntiles + KW - 1) / KW;

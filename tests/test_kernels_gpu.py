@@ -955,6 +955,31 @@ def test_attention_long_query_mask(B, H, Sq, Sk, Dh, kind):
         assert torch.all(y[:, 3] == 0)
 
 
+@pytest.mark.parametrize("mul", [1.0, 3.0, 6.0])
+@pytest.mark.parametrize("H,S,Dh", [(4, 700, 64), (26, 1340, 128), (8, 700, 128)])
+def test_attention_long_query_mask_precision(H, S, Dh, mul):
+    """Per-query masks lose no more than a softmax whose largest probability is exactly 1 has to: against
+    float64, the kernel's error is that of rounding p = exp(s - max) and the result to bf16 (both done here
+    in float64), whatever the scores' spread.  A running max that lags behind leaves the largest p inexact
+    and is 4 % (mul = 1) to 14-20 % (peaked scores) off; the sampling error of the norms is below 0.5 %."""
+    q, k, v = rnd(1, S, H * Dh, seed=181, scale=mul), rnd(1, S, H * Dh, seed=182), rnd(1, S, H * Dh, seed=183)
+    first = S // 2 - 9
+    mask = torch.ones(S, S, dtype=torch.bool)
+    mask[:first, first:] = False
+    mask[5, 7:] = False
+    split = lambda t: dev(t).double().view(S, H, Dh).transpose(0, 1).contiguous()
+    s = torch.stack([a @ b.t() for a, b in zip(split(q), split(k))]) / math.sqrt(Dh)
+    s = s.masked_fill(~dev(mask), -math.inf)
+    p = torch.exp(s - s.amax(-1, keepdim=True))
+    pr = p.to(torch.bfloat16).double()
+    vd = split(v)
+    out = lambda w: torch.stack([a @ b for a, b in zip(w / w.sum(-1, keepdim=True), vd)]).transpose(0, 1).reshape(S, H * Dh)
+    ref, rounded = out(p), out(pr).to(torch.bfloat16).double()
+    y = ops().flash_attention(dev(q), dev(k), dev(v), H, ctx_mask=dev(mask))[0].double()
+    err, want = ((t - ref).norm() / ref.norm() for t in (y, rounded))
+    assert err <= 1.02 * want, (err.item(), want.item())
+
+
 # --------------------------------------------------------------------------- rows past the end
 def _nan_tailed(rows, cols, pad, seed, scale=1.0):
     """[rows + pad, cols] bf16 whose first `rows` rows are N(0, scale) and the rest NaN: a view of
