@@ -1890,8 +1890,9 @@ static void launch_dh(const AttnArgs& a, int64_t bh, hipStream_t s) {
       // (buffer loads address a head's K and V rows with 32-bit byte offsets)
       const bool fits32 = a.Sk * a.k0_rs * 2 < ((int64_t)1 << 31) && a.Sk * a.v0_rs * 2 < ((int64_t)1 << 31);
       const int mk = a.mask_kind == FAM_MASK_NONE ? 0 : (a.mqs == 0 ? 1 : 2);
-      if (a.sk0 == a.Sk && (a.mask_kind == FAM_MASK_NONE || a.mask_kind == FAM_MASK_BOOL) && a.Sk >= 1 && fits32 && a.k0_rs >= DH &&
-          a.v0_rs >= DH) {
+      // (it masks and takes the max of unscaled scores, so the scale has to be positive)
+      if (a.sk0 == a.Sk && (a.mask_kind == FAM_MASK_NONE || a.mask_kind == FAM_MASK_BOOL) && a.Sk >= 1 && fits32 &&
+          a.k0_rs >= DH && a.v0_rs >= DH && a.scale_log2 > 0.f) {
         const int nqb = (int)((a.Sq + 127) / 128);
         const dim3 grid((unsigned)(nqb * bh));
         // a grid of at most one workgroup per CU runs each workgroup as two key groups of 4 waves

@@ -980,6 +980,24 @@ def test_attention_long_query_mask_precision(H, S, Dh, mul):
     assert err <= 1.02 * want, (err.item(), want.item())
 
 
+@pytest.mark.parametrize("scale", [0.0, -0.1, 0.05])
+@pytest.mark.parametrize("H,Sq,Sk,Dh", [(2, 131, 333, 64), (2, 131, 333, 128), (30, 1200, 257, 128)])
+def test_attention_long_any_scale(H, Sq, Sk, Dh, scale):
+    """`scale` may be any number: zero (the mean of the values that are kept), negative (the smallest product
+    wins) -- under a per-query mask, a key mask and none with a key count that leaves a partial tile."""
+    q, k, v = rnd(1, Sq, H * Dh, seed=191), rnd(1, Sk, H * Dh, seed=192), rnd(1, Sk, H * Dh, seed=193)
+    g = torch.Generator().manual_seed(194)
+    per_query, per_key = torch.rand(1, 1, Sq, Sk, generator=g) > 0.4, torch.rand(1, 1, 1, Sk, generator=g) > 0.4
+    split = lambda t: t.float().view(-1, H, Dh).transpose(0, 1).contiguous()
+    raw = torch.stack([a @ b.t() for a, b in zip(split(q), split(k))]) * scale
+    for mask in (per_query, per_key, None):
+        s = raw if mask is None else raw.masked_fill(~mask[0].expand_as(raw), -math.inf)
+        p = torch.softmax(s, -1)
+        ref = torch.stack([a @ b for a, b in zip(p, split(v))]).transpose(0, 1).reshape(1, Sq, H * Dh)
+        y = ops().attention_bshd(dev(q), dev(k), dev(v), H, mask=None if mask is None else dev(mask), scale=scale)
+        assert relerr(y, ref) <= TOL
+
+
 # --------------------------------------------------------------------------- rows past the end
 def _nan_tailed(rows, cols, pad, seed, scale=1.0):
     """[rows + pad, cols] bf16 whose first `rows` rows are N(0, scale) and the rest NaN: a view of
