@@ -219,18 +219,19 @@ __device__ __forceinline__ void row_stats(const GemmArgs& g, int64_t m0, int row
 // that belongs in its slot), which makes the fragment reads of 16 rows hit 16 distinct bank
 // groups.  Rows past M or N are past the descriptor's range and read zeros.
 template <int KW>
-__device__ __forceinline__ int panel_swz(int r) { return KW == 64 ? (r >> 1) & 7 : r & 15; }
+__device__ __forceinline__ int panel_swz(int r) { return KW == 64 || KW == 192 ? (r >> 1) & 7 : r & 15; }
 
 // ROWS rows (a multiple of 16) of the panel at byte column kb; lds and kb are wave-uniform
 template <int KW, int ROWS>
 __device__ __forceinline__ void panel_stage(__amdgpu_buffer_rsrc_t rs, uint32_t ld2, uint32_t kb, bf16* lds, int lane) {
-  constexpr int CPR = KW / 8, RPI = 512 / KW;   // chunks per row, rows per load
-  static_assert(KW == 64 || KW == 128 || KW == 256, "panel width");
+  constexpr int CPR = KW / 8, RPI = 512 / KW;   // chunks per row, rows per load (KW = 192: 2, on 48 lanes)
+  static_assert(KW == 64 || KW == 128 || KW == 192 || KW == 256, "panel width");
   const int lr = lane / CPR, lc = lane % CPR;
+  if (KW == 192 && lr >= RPI) return;
 #pragma unroll
   for (int i = 0; i < ROWS / RPI; ++i) {
     const int r = i * RPI + lr;
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void*)(lds + i * 512), 16,
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void*)(lds + i * RPI * KW), 16,
                                              (uint32_t)r * ld2 + kb + (uint32_t)((lc ^ panel_swz<KW>(r)) * 16), 0, 0, 0);
   }
 }
@@ -474,15 +475,27 @@ __global__ __launch_bounds__(NW * 64) void skinny_kernel(GemmArgs g) {
 }
 
 // skinny_staged_kernel: the same product and epilogue (no prologue, or the folded LayerNorm) with
-// staged panels, NW waves of KW columns covering K (a multiple of KW).  The row sums of the folded
-// form come from the fragments the MFMAs use; it takes 8 waves, so that a SIMD's two waves share
-// them, the plain form 4.  The DiT4DiT head (17 rows, K = 768, about 50 such launches a step): 2100 ->
-// 1934 us for a call of 4 steps.
-template <int MT, int NW, int KW, bool FOLD>
+// staged panels, NW waves staging KW columns of K each (a multiple of KW).  The row sums of the
+// folded form come from the fragments the MFMAs use; it takes 8 waves, so that a SIMD's two waves
+// share them, the plain form 4, or 8 for 16 rows of K up to 2048.  The DiT4DiT head (17 rows,
+// K = 768, about 50 such launches a step): 2100 -> 1962 us for a call of 4
+// steps.
+// The sums keep skinny_kernel's grouping, and so its bits: NG runs of G k-steps (its waves' shares
+// of K), each an accumulator of its own, added in order.  Where a wave's runs are not its own panel
+// (the folded form's K = 768 is 8 runs of 3 k-steps and 6 panels of 4), the panels are shared behind
+// a barrier.
+template <int MT, int NW, int KW, int G, bool FOLD>
 __global__ __launch_bounds__(NW * 64) void skinny_staged_kernel(GemmArgs g) {
-  constexpr bool WD = MT == 4 && NW * KW == 1024;   // 80 rows x 2 KB would be the whole LDS
+  constexpr int NG = FOLD || NW == 4 ? 8 : 16, GPW = NG / NW, SP = KW / 32;   // runs, per wave; k-steps per panel
+  constexpr bool OWN = G * GPW == SP;
+  constexpr int NP = G * NG / SP;                   // panels
+  constexpr bool WD = MT == 4 && NP * KW == 1024;   // 80 rows x 2 KB would be the whole LDS
+  static_assert(NP <= NW && (OWN || !WD) && (!FOLD || GPW == 1), "skinny_staged_kernel: split");
   constexpr int MR = MT * 16, ROWS = MR + (WD ? 0 : 16);
-  __shared__ __attribute__((aligned(1024))) bf16 sm[NW][ROWS * KW];
+  static_assert(!OWN || GPW * MT * 4 * 20 * 8 <= ROWS * KW, "a wave's accumulators fit its panel");
+  __shared__ __attribute__((aligned(1024))) bf16 sm[NP][ROWS * KW];
+  constexpr int LP = OWN ? 20 : 16;   // 16-byte slots from one lane group of a tile to the next (20: no bank conflicts)
+  __shared__ f32x4 s_acc[OWN ? 1 : NG * MT * 64];
   __shared__ float2 s_st[FOLD ? NW : 1][MR];
   __shared__ float s_piv[MR];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -490,17 +503,16 @@ __global__ __launch_bounds__(NW * 64) void skinny_staged_kernel(GemmArgs g) {
   const int M = (int)g.M, N = (int)g.N, K = (int)g.K;
   const int n0 = blockIdx.x * 16, k0 = wave * KW;
   const uint32_t lda2 = (uint32_t)g.lda * 2u, ldw2 = (uint32_t)g.ldw * 2u, kb = (uint32_t)k0 * 2u;
-  bf16* const my = &sm[wave][0];
-  bf16x8 wf[WD ? KW / 32 : 1];
-  if (k0 < K) {
+  bf16x8 wf[WD ? SP : 1];
+  if (k0 < K) {   // (then wave < NP)
     const auto rw = buffer_rsrc(g.w + (int64_t)n0 * g.ldw, (uint32_t)min(16, N - n0) * ldw2);
     if constexpr (WD) {
 #pragma unroll
-      for (int s = 0; s < KW / 32; ++s) wf[s] = buffer_load8(rw, (uint32_t)l16 * ldw2 + kb + (uint32_t)(4 * s + lg) * 16u);
+      for (int s = 0; s < SP; ++s) wf[s] = buffer_load8(rw, (uint32_t)l16 * ldw2 + kb + (uint32_t)(4 * s + lg) * 16u);
     } else {
-      panel_stage<KW, 16>(rw, ldw2, kb, my + MR * KW, lane);
+      panel_stage<KW, 16>(rw, ldw2, kb, &sm[wave][MR * KW], lane);
     }
-    panel_stage<KW, MR>(buffer_rsrc(g.a, (uint32_t)M * lda2), lda2, kb, my, lane);
+    panel_stage<KW, MR>(buffer_rsrc(g.a, (uint32_t)M * lda2), lda2, kb, &sm[wave][0], lane);
   }
   // each thread's epilogue operands, and the rows' pivots, in flight with the panels
   constexpr int EPT = (MR * 16 + NW * 64 - 1) / (NW * 64);
@@ -520,28 +532,51 @@ __global__ __launch_bounds__(NW * 64) void skinny_staged_kernel(GemmArgs g) {
     }
   }
   __builtin_amdgcn_sched_barrier(0);
-  f32x4 acc[MT];
+  f32x4 acc[GPW][MT];
 #pragma unroll
-  for (int i = 0; i < MT; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-  if (k0 < K) {
-    panel_wait();
+  for (int r = 0; r < GPW; ++r)
 #pragma unroll
-    for (int s = 0; s < KW / 32; ++s) {
-      const bf16x8 w = WD ? wf[s] : panel_frag<KW>(my, MR, s, l16, lg);
+    for (int i = 0; i < MT; ++i) acc[r][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  auto step = [&](const bf16* pan, int s, bf16x8 w, f32x4 (&ac)[MT]) {
 #pragma unroll
-      for (int i = 0; i < MT; ++i) {
-        const bf16x8 af = panel_frag<KW>(my, 16 * i, s, l16, lg);
-        acc[i] = mfma16(w, af, acc[i]);
-        if constexpr (FOLD) {
+    for (int i = 0; i < MT; ++i) {
+      const bf16x8 af = panel_frag<KW>(pan, 16 * i, s, l16, lg);
+      ac[i] = mfma16(w, af, ac[i]);
+      if constexpr (FOLD) {
 #pragma unroll
-          for (int e = 0; e < 8; ++e) {
-            const float d = to_f(af[e]) - piv[i];
-            s1[i] += d;
-            s2[i] += d * d;
-          }
+        for (int e = 0; e < 8; ++e) {
+          const float d = to_f(af[e]) - piv[i];
+          s1[i] += d;
+          s2[i] += d * d;
         }
       }
     }
+  };
+  if constexpr (OWN) {
+    if (k0 < K) {
+      const bf16* pan = &sm[wave][0];
+      panel_wait();
+#pragma unroll
+      for (int r = 0; r < GPW; ++r)
+#pragma unroll
+        for (int j = 0; j < G; ++j) {
+          const int s = r * G + j;
+          step(pan, s, WD ? wf[s] : panel_frag<KW>(pan, MR, s, l16, lg), acc[r]);
+        }
+    }
+  } else {
+    panel_wait();
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < GPW; ++r)
+#pragma unroll
+      for (int j = 0; j < G; ++j) {
+        const int s = (wave * GPW + r) * G + j;
+        if (32 * s < K) {   // uniform
+          const bf16* pan = &sm[s / SP][0];
+          step(pan, s % SP, panel_frag<KW>(pan, MR, s % SP, l16, lg), acc[r]);
+        }
+      }
   }
   if constexpr (FOLD) {
 #pragma unroll
@@ -554,21 +589,27 @@ __global__ __launch_bounds__(NW * 64) void skinny_staged_kernel(GemmArgs g) {
       }
     }
   }
-  // the accumulators in the wave's own panel: lane (lg, l16) holds out[16 i + l16][n0 + 4 lg + e]
+  // the runs' accumulators (in the wave's own panel, which only it reads): lane (lg, l16) holds
+  // out[16 i + l16][n0 + 4 lg + e]
+  auto run_acc = [&](int q) {
+    return OWN ? reinterpret_cast<f32x4*>(&sm[q / GPW][0]) + (q % GPW) * MT * 4 * LP : s_acc + q * MT * 4 * LP;
+  };
   asm volatile("" ::: "memory");
 #pragma unroll
-  for (int i = 0; i < MT; ++i) *reinterpret_cast<f32x4*>(my + (i * 64 + lane) * 8) = acc[i];
+  for (int r = 0; r < GPW; ++r)
+#pragma unroll
+    for (int i = 0; i < MT; ++i) run_acc(wave * GPW + r)[i * 4 * LP + lg * LP + l16] = acc[r][i];
   __syncthreads();
 #pragma unroll
   for (int u = 0; u < EPT; ++u) {
     const int t = tid + u * NW * 64, mr = t >> 4, c = t & 15, n = n0 + c;
     if (t >= MR * 16 || mr >= M || n >= N) continue;
-    const int at = ((mr >> 4) * 64 + (c >> 2) * 16 + (mr & 15)) * 4 + (c & 3);
-    float p[NW], v = 0.f;
+    const int at = (((mr >> 4) * 4 + (c >> 2)) * LP + (mr & 15)) * 4 + (c & 3);
+    float p[NG], v = 0.f;
 #pragma unroll
-    for (int w = 0; w < NW; ++w) p[w] = reinterpret_cast<const float*>(&sm[w][0])[at];
+    for (int q = 0; q < NG; ++q) p[q] = reinterpret_cast<const float*>(run_acc(q))[at];
 #pragma unroll
-    for (int w = 0; w < NW; ++w) v += p[w];
+    for (int q = 0; q < NG; ++q) v += p[q];
     if constexpr (FOLD) {
       float t1 = 0.f, t2 = 0.f;
 #pragma unroll
@@ -1539,21 +1580,30 @@ static bool panel_ok(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldw, 
 template <int MT>
 static bool launch_skinny_staged(const GemmArgs& a, int pro, hipStream_t s) {
   const dim3 grid((unsigned)(round_up(a.N, 16) / 16));
-  auto ok = [&](int kw) { return panel_ok(a.M, a.N, a.K, a.lda, a.ldw, kw); };
-  if (pro == FAM_PRO_LN_FOLDED) {
-    if (a.K <= 512 && ok(64)) FAM_LAUNCH((skinny_staged_kernel<MT, 8, 64, true>), grid, dim3(512), 0, s, a);
-    else if (a.K > 512 && a.K <= 1024 && ok(128)) FAM_LAUNCH((skinny_staged_kernel<MT, 8, 128, true>), grid, dim3(512), 0, s, a);
-    else return false;
+  const bool fold = pro == FAM_PRO_LN_FOLDED;
+  if ((pro != FAM_PRO_NONE && !fold) || a.K > (fold || MT > 1 ? 1024 : 2048)) return false;
+  const int kw = fold ? (a.K <= 512 ? 64 : 128) : (a.K <= 256 ? 64 : a.K <= 512 ? 128 : 256);
+  if (!panel_ok(a.M, a.N, a.K, a.lda, a.ldw, kw)) return false;
+  const int runs = a.K <= 1024 ? 8 : 16, per = (int)(a.K / 32 + runs - 1) / runs;   // skinny_kernel's k-steps per wave
+  if (fold) {
+    if (per == 1) FAM_LAUNCH((skinny_staged_kernel<MT, 8, 64, 1, true>), grid, dim3(512), 0, s, a);
+    else if (per == 2) FAM_LAUNCH((skinny_staged_kernel<MT, 8, 64, 2, true>), grid, dim3(512), 0, s, a);
+    else if (per == 3) FAM_LAUNCH((skinny_staged_kernel<MT, 8, 128, 3, true>), grid, dim3(512), 0, s, a);
+    else FAM_LAUNCH((skinny_staged_kernel<MT, 8, 128, 4, true>), grid, dim3(512), 0, s, a);
     return true;
   }
-  if (pro != FAM_PRO_NONE) return false;
-  if (a.K <= 256 && ok(64)) FAM_LAUNCH((skinny_staged_kernel<MT, 4, 64, false>), grid, dim3(256), 0, s, a);
-  else if (a.K > 256 && a.K <= 512 && ok(128)) FAM_LAUNCH((skinny_staged_kernel<MT, 4, 128, false>), grid, dim3(256), 0, s, a);
-  else if (a.K > 512 && a.K <= 1024 && ok(256)) FAM_LAUNCH((skinny_staged_kernel<MT, 4, 256, false>), grid, dim3(256), 0, s, a);
-  else if (MT == 1 && a.K > 1024 && a.K <= 2048 && ok(256)) {
-    // (16 rows of activations and 16 of weights x 4 KB: 128 KB)
-    if constexpr (MT == 1) FAM_LAUNCH((skinny_staged_kernel<1, 8, 256, false>), grid, dim3(512), 0, s, a);
-  } else return false;
+  if constexpr (MT == 1) {
+    if (a.K > 1024) {   // (16 rows of activations and 16 of weights x 4 KB: 128 KB)
+      if (per == 3 && a.K % 192 == 0) FAM_LAUNCH((skinny_staged_kernel<1, 8, 192, 3, false>), grid, dim3(512), 0, s, a);
+      else if (per == 3) FAM_LAUNCH((skinny_staged_kernel<1, 8, 256, 3, false>), grid, dim3(512), 0, s, a);
+      else FAM_LAUNCH((skinny_staged_kernel<1, 8, 256, 4, false>), grid, dim3(512), 0, s, a);
+      return true;
+    }
+  }
+  if (per == 1) FAM_LAUNCH((skinny_staged_kernel<MT, 4, 64, 1, false>), grid, dim3(256), 0, s, a);
+  else if (per == 2) FAM_LAUNCH((skinny_staged_kernel<MT, 4, 128, 2, false>), grid, dim3(256), 0, s, a);
+  else if (per == 3) FAM_LAUNCH((skinny_staged_kernel<MT, 4, 192, 3, false>), grid, dim3(256), 0, s, a);
+  else FAM_LAUNCH((skinny_staged_kernel<MT, 4, 256, 4, false>), grid, dim3(256), 0, s, a);
   return true;
 }
 
@@ -2120,11 +2170,12 @@ static void launch_final_steps(const FinalArgs& a, int steps, hipStream_t s) {
 
 template <int MT>
 static void launch_final(const FinalArgs& a, hipStream_t s) {
-  // K <= 1024 in whole panels (the narrowest of 64, 128, 256 columns that four waves cover K
-  // with): staged.  Otherwise the register form:
+  // 128 < K <= 1024 in whole panels (the narrowest of 64, 128, 256 columns that four waves cover K
+  // with): staged.  Otherwise the register form (K = 64 and 128, one k-step per wave: 2.16 us at
+  // 17 rows against 2.23 staged, and sums of their own):
   const int kw = a.K <= 256 ? 64 : a.K <= 512 ? 128 : 256;
-  if (a.K <= 1024 && panel_ok(a.M, a.N, a.K, a.lda, a.ldw, kw)) {
-    const dim3 grid((unsigned)((a.N + 15) / 16));
+  const dim3 grid((unsigned)((a.N + 15) / 16));
+  if (a.K > 128 && a.K <= 1024 && panel_ok(a.M, a.N, a.K, a.lda, a.ldw, kw)) {
     if (kw == 64) FAM_LAUNCH((final_staged_kernel<MT, 64>), grid, dim3(256), 0, s, a);
     else if (kw == 128) FAM_LAUNCH((final_staged_kernel<MT, 128>), grid, dim3(256), 0, s, a);
     else FAM_LAUNCH((final_staged_kernel<MT, 256>), grid, dim3(256), 0, s, a);

@@ -1074,3 +1074,60 @@ def test_staged_panels_small_m(M, N, K):
         assert ((y - rb).abs() <= lim + rb.abs() * 2.0 ** -8 + 1e-30).all()
         sq = torch.nn.functional.pad(y.square(), (0, -N % 16)).reshape(M, -1, 16).sum(-1)
         assert torch.allclose(ss.double().cpu(), sq, rtol=1e-5, atol=1e-12)
+
+
+@pytest.mark.parametrize("K", [64, 192, 256, 384, 512, 768, 1024, 1280, 1536, 1792, 2048])
+@pytest.mark.parametrize("M", [1, 16, 17, 40, 64])
+def test_skinny_sums_are_grouped_alike(M, K):
+    """A skinny product is the sum of 8 runs of K (16 above 1024), each a whole number of 32-wide k-steps,
+    added in fp32 in their order -- whichever kernel serves the call.  Every run's own sum is 24 bits from
+    three bf16 values (exact in any order), so the result tells the grouping to the last bit."""
+    steps, runs = K // 32, 8 if K <= 1024 else 16
+    per = -(-steps // runs) * 32
+    g = torch.Generator().manual_seed(7)
+    a = torch.zeros(M, K)
+    total = torch.zeros(M)
+    for lo in range(0, K, per):
+        e = torch.randint(-6, 7, (M,), generator=g).float()
+        at = torch.stack([torch.randperm(min(per, K - lo), generator=g)[:3] for _ in range(M)]) + lo
+        run = torch.zeros(M)
+        for j, sc in enumerate((2.0 ** 16, 2.0 ** 8, 1.0)):
+            v = torch.randint(-255, 256, (M,), generator=g).float() * sc * 2.0 ** e
+            a[torch.arange(M), at[:, j]] = v
+            run = run + v
+        total = total + run                              # fp32, in order
+    ad, w = dev(a.to(torch.bfloat16)), torch.ones(48, K, dtype=torch.bfloat16, device="cuda")
+    assert torch.equal(ad.float().cpu(), a)
+    y = torch.empty(M, 48, dtype=torch.float32, device="cuda")
+    ops().gemm(ad, w, None, y, out_f32=True)
+    assert torch.equal(y.cpu(), total[:, None].expand(M, 48))
+
+
+@pytest.mark.parametrize("K,per", [(128, 32), (192, 64), (256, 64), (512, 128), (1024, 256)])
+@pytest.mark.parametrize("M", [1, 17, 64])
+def test_gemm_final_sums_are_grouped_alike(M, K, per):
+    """fam_gemm_final adds the sums of its waves' shares of K in order: 2^24 in the first and 1 in each later
+    one stays 2^24 in fp32 (ties to even), where two of the later ones summed first would show as 2."""
+    a = torch.zeros(M, K)
+    a[:, 0] = 2.0 ** 24
+    a[:, per + 1::per] = 1.0
+    y = ops().gemm_final(dev(a.to(torch.bfloat16)), torch.ones(32, K, dtype=torch.bfloat16, device="cuda"),
+                         torch.full((32,), -2.0 ** 24, dtype=torch.bfloat16, device="cuda"))
+    assert not y.any()
+
+
+@pytest.mark.parametrize("K", [64, 128, 192, 320, 512, 640, 768, 896, 1024])
+@pytest.mark.parametrize("M", [1, 16, 17, 50, 64])
+def test_gemm_folded_layernorm_staged(M, K):
+    """Every staged form of the folded LayerNorm: 16-, 32- and 64-row tiles, panels of 64 and 128 columns, the
+    wave's own and shared ones.  Against float64; the row sums and the product are fp32 sums of at most
+    K terms, |x - pivot| <= 8 here, so their error is below the bf16 rounding of the result (2^-9) by far."""
+    from fam import _capi
+    N = 200
+    x, w, b = rnd(M, K, seed=201), rnd(N, K, seed=202, scale=0.05), rnd(N, seed=203)
+    xd, wd = x.double(), w.double()
+    ref = torch.nn.functional.layer_norm(xd, (K,), eps=1e-6) @ wd.t() + b.double()
+    y = torch.empty(M, N, dtype=torch.bfloat16, device="cuda")
+    ops().gemm(dev(x), dev(w), dev(b), y, prologue=_capi.FAM_PRO_LN_FOLDED, pro_w=dev(wd.sum(1).float()), pro_eps=1e-6)
+    err = (y.double().cpu() - ref).abs()
+    assert (err <= 2.0 ** -8 * ref.abs() + 1e-4 * ref.abs().max()).all(), err.max().item()
