@@ -221,19 +221,27 @@ __device__ __forceinline__ void row_stats(const GemmArgs& g, int64_t m0, int row
 template <int KW>
 __device__ __forceinline__ int panel_swz(int r) { return KW == 64 || KW == 192 ? (r >> 1) & 7 : r & 15; }
 
-// ROWS rows (a multiple of 16) of the panel at byte column kb; lds and kb are wave-uniform
+// ROWS rows (a multiple of 16) of the panel at byte column kb; lds, kb and rows are wave-uniform.
+// Eights of rows that lie past `rows` are left out: what their LDS holds only reaches outputs that
+// are never stored, and their loads made 17 rows as dear as 32 (fam_gemm_final, K = 1024, N = 1024: 17
+// rows 4.27 -> 4.05 us, 33 rows 5.21 -> 4.93).
 template <int KW, int ROWS>
-__device__ __forceinline__ void panel_stage(__amdgpu_buffer_rsrc_t rs, uint32_t ld2, uint32_t kb, bf16* lds, int lane) {
+__device__ __forceinline__ void panel_stage(__amdgpu_buffer_rsrc_t rs, uint32_t ld2, uint32_t kb, bf16* lds, int lane,
+                                            int rows) {
   constexpr int CPR = KW / 8, RPI = 512 / KW;   // chunks per row, rows per load (KW = 192: 2, on 48 lanes)
   static_assert(KW == 64 || KW == 128 || KW == 192 || KW == 256, "panel width");
   const int lr = lane / CPR, lc = lane % CPR;
   if (KW == 192 && lr >= RPI) return;
 #pragma unroll
-  for (int i = 0; i < ROWS / RPI; ++i) {
-    const int r = i * RPI + lr;
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void*)(lds + i * RPI * KW), 16,
-                                             (uint32_t)r * ld2 + kb + (uint32_t)((lc ^ panel_swz<KW>(r)) * 16), 0, 0, 0);
-  }
+  for (int o = 0; o < ROWS / 8; ++o)
+    if (8 * o < rows) {
+#pragma unroll
+      for (int i = o * 8 / RPI; i < (o + 1) * 8 / RPI; ++i) {
+        const int r = i * RPI + lr;
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void*)(lds + i * RPI * KW), 16,
+                                                 (uint32_t)r * ld2 + kb + (uint32_t)((lc ^ panel_swz<KW>(r)) * 16), 0, 0, 0);
+      }
+    }
 }
 // the fragment of rows r0 .. r0 + 15 (r0 a multiple of 16), k-step s
 template <int KW>
@@ -478,7 +486,7 @@ __global__ __launch_bounds__(NW * 64) void skinny_kernel(GemmArgs g) {
 // staged panels, NW waves staging KW columns of K each (a multiple of KW).  The row sums of the
 // folded form come from the fragments the MFMAs use; it takes 8 waves, so that a SIMD's two waves
 // share them, the plain form 4, or 8 for 16 rows of K up to 2048.  The DiT4DiT head (17 rows,
-// K = 768, about 50 such launches a step): 2100 -> 1962 us for a call of 4
+// K = 768, about 50 such launches a step): 2100 -> 1943 us for a call of 4
 // steps.
 // The sums keep skinny_kernel's grouping, and so its bits: NG runs of G k-steps (its waves' shares
 // of K), each an accumulator of its own, added in order.  Where a wave's runs are not its own panel
@@ -510,9 +518,9 @@ __global__ __launch_bounds__(NW * 64) void skinny_staged_kernel(GemmArgs g) {
 #pragma unroll
       for (int s = 0; s < SP; ++s) wf[s] = buffer_load8(rw, (uint32_t)l16 * ldw2 + kb + (uint32_t)(4 * s + lg) * 16u);
     } else {
-      panel_stage<KW, 16>(rw, ldw2, kb, &sm[wave][MR * KW], lane);
+      panel_stage<KW, 16>(rw, ldw2, kb, &sm[wave][MR * KW], lane, 16);
     }
-    panel_stage<KW, MR>(buffer_rsrc(g.a, (uint32_t)M * lda2), lda2, kb, &sm[wave][0], lane);
+    panel_stage<KW, MR>(buffer_rsrc(g.a, (uint32_t)M * lda2), lda2, kb, &sm[wave][0], lane, M);
   }
   // each thread's epilogue operands, and the rows' pivots, in flight with the panels
   constexpr int EPT = (MR * 16 + NW * 64 - 1) / (NW * 64);
@@ -727,9 +735,9 @@ __global__ __launch_bounds__(256) void partial_staged_kernel(PartArgs g) {
 #pragma unroll
       for (int s = 0; s < KW / 32; ++s) wf[s] = buffer_load8(rw, (uint32_t)l16 * ldw2 + kb + (uint32_t)(4 * s + lg) * 16u);
     } else {
-      panel_stage<KW, 16>(rw, ldw2, kb, &sm[wave][16 * MT * KW], lane);
+      panel_stage<KW, 16>(rw, ldw2, kb, &sm[wave][16 * MT * KW], lane, 16);
     }
-    panel_stage<KW, 16 * MT>(buffer_rsrc(g.a, (uint32_t)M * lda2), lda2, kb, &sm[wave][0], lane);
+    panel_stage<KW, 16 * MT>(buffer_rsrc(g.a, (uint32_t)M * lda2), lda2, kb, &sm[wave][0], lane, M);
     panel_wait();
     panel_mfma<MT, KW, WD>(&sm[wave][0], wf, l16, lg, acc);
   }
@@ -1080,9 +1088,9 @@ __global__ __launch_bounds__(256) void final_staged_kernel(FinalArgs g) {
 #pragma unroll
       for (int s = 0; s < KW / 32; ++s) wf[s] = buffer_load8(rw, (uint32_t)l16 * ldw2 + kb + (uint32_t)(4 * s + lg) * 16u);
     } else {
-      panel_stage<KW, 16>(rw, ldw2, kb, &sm[wave][16 * MT * KW], lane);
+      panel_stage<KW, 16>(rw, ldw2, kb, &sm[wave][16 * MT * KW], lane, 16);
     }
-    panel_stage<KW, 16 * MT>(buffer_rsrc(g.a, (uint32_t)M * lda2), lda2, kb, &sm[wave][0], lane);
+    panel_stage<KW, 16 * MT>(buffer_rsrc(g.a, (uint32_t)M * lda2), lda2, kb, &sm[wave][0], lane, M);
     panel_wait();
     panel_mfma<MT, KW, WD>(&sm[wave][0], wf, l16, lg, acc);
   }
@@ -1585,6 +1593,15 @@ static bool launch_skinny_staged(const GemmArgs& a, int pro, hipStream_t s) {
   const int kw = fold ? (a.K <= 512 ? 64 : 128) : (a.K <= 256 ? 64 : a.K <= 512 ? 128 : 256);
   if (!panel_ok(a.M, a.N, a.K, a.lda, a.ldw, kw)) return false;
   const int runs = a.K <= 1024 ? 8 : 16, per = (int)(a.K / 32 + runs - 1) / runs;   // skinny_kernel's k-steps per wave
+  // Panels of K > 512 leave room for one workgroup per CU, so where the grid takes several rounds
+  // the register form, which shares a CU, is ahead if most of the tile's rows are padding (its
+  // loads of those hit the cache).  Register : staged us at N = 9216, K = 1024: plain 17 rows 9.5 :
+  // 9.9, 20 rows 9.9 : 9.7; folded 1 row 7.0 : 7.4, 8 rows 8.2 : 7.7, 17 rows 11.6 : 12.1, 32 rows
+  // 13.9 : 13.4; folded K = 768, whose panels are shared, 17 rows 10.4 : 11.6, 32 rows 12.2 : 12.9.
+  const int64_t wgs = grid.x, cus = fam_host::device_cus();
+  if (fold && a.K > 512 && wgs > 2 * cus && a.M <= (per == 3 ? 8 : 4)) return false;
+  if (fold && a.K > 512 && MT == 2 && wgs > (per == 3 ? 1 : 2) * cus && a.M <= (per == 3 ? 32 : 28)) return false;
+  if (!fold && a.K > 768 && MT == 2 && wgs > 2 * cus && a.M < 20) return false;
   if (fold) {
     if (per == 1) FAM_LAUNCH((skinny_staged_kernel<MT, 8, 64, 1, true>), grid, dim3(512), 0, s, a);
     else if (per == 2) FAM_LAUNCH((skinny_staged_kernel<MT, 8, 64, 2, true>), grid, dim3(512), 0, s, a);
@@ -2041,12 +2058,25 @@ extern "C" int fam_gemm_partial_splits(int64_t M, int64_t N, int64_t K) {
   return M > 128 && st >= 0 ? 0 : sp;
 }
 
+// Panels of 256 columns leave room for one workgroup per CU; where a grid takes several rounds, the
+// register form, which shares a CU, is ahead of them if most of the tile's rows are padding.
+// Register : staged us, fam_gemm_final at K = 1024: N = 9216, 17 rows 9.3 : 10.2, 28 rows 10.6 :
+// 10.6, 32 rows 11.1 : 10.7; N = 14336, 17 rows 11.5 : 13.5, 28 rows 13.4 : 14.1, 32 rows 14.1 :
+// 14.1.  fam_gemm_partial: 2048 x 8192 (1024 workgroups) 17 rows 12.5 : 14.8, 33 rows 16.4 : 17.3, 40
+// rows 17.7 : 17.5; 3072 x 14336 (2688) 1 row 18.4 : 21.3, 8 rows 21.9 : 21.3.
+static bool staged_crowded(int64_t M, int steps, int64_t wgs) {
+  const int64_t cus = fam_host::device_cus();
+  return steps == 8 && ((wgs > 2 * cus && M > 16 && M <= 28) || (wgs > 3 * cus && M > 32 && M <= 36) ||
+                        (wgs > 8 * cus && M <= 4));
+}
+
 template <int MT>
 static void launch_partial(const PartArgs& a, int steps, int splits, hipStream_t s) {
   const dim3 grid((unsigned)((a.N + 15) / 16), (unsigned)splits);
   if constexpr (MT <= 4) {
     // (one k-step per wave is a 64-byte piece per row either way)
-    if (steps > 1 && panel_ok(a.M, a.N, a.K, a.lda, a.ldw, 32 * steps)) {
+    if (steps > 1 && panel_ok(a.M, a.N, a.K, a.lda, a.ldw, 32 * steps) &&
+        !staged_crowded(a.M, steps, (int64_t)grid.x * grid.y)) {
       if (steps == 2) FAM_LAUNCH((partial_staged_kernel<MT, 64>), grid, dim3(256), 0, s, a);
       else if (steps == 4) FAM_LAUNCH((partial_staged_kernel<MT, 128>), grid, dim3(256), 0, s, a);
       else FAM_LAUNCH((partial_staged_kernel<MT, 256>), grid, dim3(256), 0, s, a);
@@ -2175,7 +2205,7 @@ static void launch_final(const FinalArgs& a, hipStream_t s) {
   // 17 rows against 2.23 staged, and sums of their own):
   const int kw = a.K <= 256 ? 64 : a.K <= 512 ? 128 : 256;
   const dim3 grid((unsigned)((a.N + 15) / 16));
-  if (a.K > 128 && a.K <= 1024 && panel_ok(a.M, a.N, a.K, a.lda, a.ldw, kw)) {
+  if (a.K > 128 && a.K <= 1024 && panel_ok(a.M, a.N, a.K, a.lda, a.ldw, kw) && !staged_crowded(a.M, kw / 32, grid.x)) {
     if (kw == 64) FAM_LAUNCH((final_staged_kernel<MT, 64>), grid, dim3(256), 0, s, a);
     else if (kw == 128) FAM_LAUNCH((final_staged_kernel<MT, 128>), grid, dim3(256), 0, s, a);
     else FAM_LAUNCH((final_staged_kernel<MT, 256>), grid, dim3(256), 0, s, a);

@@ -1131,3 +1131,38 @@ def test_gemm_folded_layernorm_staged(M, K):
     ops().gemm(dev(x), dev(w), dev(b), y, prologue=_capi.FAM_PRO_LN_FOLDED, pro_w=dev(wd.sum(1).float()), pro_eps=1e-6)
     err = (y.double().cpu() - ref).abs()
     assert (err <= 2.0 ** -8 * ref.abs() + 1e-4 * ref.abs().max()).all(), err.max().item()
+
+
+@pytest.mark.parametrize("M", [1, 4, 8, 17, 19, 20, 28, 32, 33])
+@pytest.mark.parametrize("K", [768, 1024])
+def test_small_m_routes_agree(M, K):
+    """Where a grid takes several rounds over the CUs, tiles that are mostly padding leave the staged panels
+    for the register kernels: the same product in pieces of 1024 columns (staged) has the same bits."""
+    from fam import _capi
+    N = 9216 + 16
+    a, w, b = dev(rnd(M, K, seed=211)), dev(rnd(N, K, seed=212, scale=0.02)), dev(rnd(N, seed=213))
+    cs = w.float().sum(1)
+
+    def plain(w, b, c):
+        y = torch.empty(M, w.shape[0], dtype=torch.float32, device="cuda")
+        ops().gemm(a, w, b, y, out_f32=True)
+        return y
+
+    def folded(w, b, c):
+        y = torch.empty(M, w.shape[0], dtype=torch.float32, device="cuda")
+        ops().gemm(a, w, b, y, out_f32=True, prologue=_capi.FAM_PRO_LN_FOLDED, pro_w=c)
+        return y
+    final = lambda w, b, c: ops().gemm_final(a, w, b)
+    for f in (plain, folded, final):
+        whole = f(w, b, cs)
+        for n0 in range(0, N, 1024):
+            n1 = min(N, n0 + 1024)
+            assert torch.equal(whole[:, n0:n1], f(w[n0:n1], b[n0:n1], cs[n0:n1].contiguous())), (f, n0)
+
+
+@pytest.mark.parametrize("M,Mfull,N,K", [(17, 32, 3072, 4096), (28, 32, 2048, 8192), (33, 40, 2048, 8192), (4, 8, 3072, 14336)])
+def test_partial_routes_agree(M, Mfull, N, K):
+    """The planes of M rows (register kernel) are the first M rows of those of Mfull (staged)."""
+    a, w = dev(rnd(Mfull, K, seed=221)), dev(rnd(N, K, seed=222, scale=0.02))
+    (few, s0), (full, s1) = ops().gemm_partial(a[:M], w), ops().gemm_partial(a, w)
+    assert s0 == s1 and torch.equal(few, full[:, :M])
