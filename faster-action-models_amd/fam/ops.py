@@ -490,7 +490,8 @@ def _attention_op(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, mask: Optio
 
 
 def _attention(q, k, v, mask, num_heads: int, scale, k_prefix, v_prefix, num_splits: int) -> torch.Tensor:
-    if _plain(q, k, v, mask, k_prefix, v_prefix):
+    # (any other scale, a text say, is the operator's schema to convert or refuse)
+    if (scale is None or isinstance(scale, (float, int))) and _plain(q, k, v, mask, k_prefix, v_prefix):
         return _attention_launch(q, k, v, num_heads, mask, scale, k_prefix, v_prefix, None, num_splits, None)
     return torch.ops.fam.attention(q, k, v, mask, num_heads, scale, k_prefix, v_prefix, num_splits)
 

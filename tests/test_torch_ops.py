@@ -373,3 +373,17 @@ def test_rope_tables_of_a_conjugated_table_are_its_own(first):
     for v in order + order:
         cos, sin, _, _ = ops.rope_tables(v, "cat", dev)
         assert not cos.is_neg() and torch.equal(cos[:, :8], v.reshape(8, 16)[:, :8].clone())
+
+
+def test_attention_scale_is_a_number(monkeypatch):
+    """A scale that is no number is refused by the operator's schema, also for a plain call."""
+    seen = []
+    monkeypatch.setattr(ops, "_attention_launch", lambda *a: seen.append(a[5]))
+    q = torch.zeros(1, 4, 64, dtype=torch.bfloat16)
+    for scale in ("0.5", b"1", [0.5], 1j):
+        with pytest.raises(RuntimeError, match="scale"):
+            ops.attention_bshd(q, q, q, 1, scale=scale)
+    assert not seen
+    for scale in (None, 0.5, 1):
+        ops.attention_bshd(q, q, q, 1, scale=scale)
+    assert seen == [None, 0.5, 1]
