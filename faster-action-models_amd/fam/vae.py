@@ -134,7 +134,9 @@ class FusedWanVAEEncoder:
             w = w.permute(0, 2, 3, 1).reshape(co, 9 * ci)
             out = torch.zeros(co, _kpad(9 * ci), dtype=_BF16, device=dev)
             out[:, :9 * ci] = w.to(_BF16)
-            return out.contiguous(), P(bn).to(_BF16).contiguous()
+            b = P(bn).to(_BF16).contiguous()
+            # (fam_conv3x3 reads the bias in vectors; a view into a larger buffer may lie anywhere)
+            return out.contiguous(), b if b.data_ptr() % 16 == 0 else b.clone()
 
         def conv1x1(wn, bn, rows=None):
             w = P(wn).float().reshape(P(wn).shape[0], -1)

@@ -237,3 +237,20 @@ def test_cosmos_shapes_and_rope_tables_match_oracle():
         c1, s1 = cosmos.cosmos_rope_tables(cfg, 2, 32, 32, fps, "cpu")
         c2, s2 = O.cosmos_rope_tables(ocfg, 2, 32, 32, fps)
         assert torch.equal(c1, c2) and torch.equal(s1, s2)
+
+
+def test_vae_convolution_biases_are_aligned():
+    """bf16 biases that are views at odd addresses of a larger buffer (a flat parameter store): the plan's
+    3x3 convolutions, which fam_conv3x3 runs on 8-byte aligned biases only, hold aligned copies of them."""
+    from fam import vae
+    cfg = vae.WanVaeConfig(dim=32)
+    params = {}
+    for n, s in vae.encoder_param_shapes(cfg).items():
+        flat = torch.arange(1 + torch.Size(s).numel()).to(torch.bfloat16)
+        params[n] = flat[1:].view(s) if n.endswith("bias") else flat[1:].clone().view(s)
+    assert any(p.data_ptr() % 8 for n, p in params.items() if n.endswith("bias"))
+    enc = vae.FusedWanVAEEncoder(cfg, params, height=64, width=64, device="cpu")
+    convs = [d for d in enc._descs if d.K >= 9 * 32]
+    assert len(convs) >= 20 and all(d.bias and d.bias % 16 == 0 for d in convs)
+    head = [t for t in enc._keep if t.dim() == 1 and t.shape == (2 * cfg.z_dim,)]
+    assert any(torch.equal(t, params["encoder.head.2.bias"]) for t in head)
