@@ -45,7 +45,10 @@ _PLAIN_TYPES = (torch.Tensor, torch.nn.Parameter)
 
 
 def _stream(t: torch.Tensor) -> int:
-    return torch._C._cuda_getCurrentRawStream(t.get_device())
+    dev = t.get_device()
+    if dev < 0:   # (which the getter would take for the current device, and the launch for device memory)
+        raise ValueError(f"expected a tensor on a HIP device (got {t.device})")
+    return torch._C._cuda_getCurrentRawStream(dev)
 
 
 def _plain(*tensors) -> bool:

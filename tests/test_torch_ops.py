@@ -387,3 +387,18 @@ def test_attention_scale_is_a_number(monkeypatch):
     for scale in (None, 0.5, 1):
         ops.attention_bshd(q, q, q, 1, scale=scale)
     assert seen == [None, 0.5, 1]
+
+
+def test_host_tensors_never_reach_a_launch(monkeypatch):
+    """gemm and rowop, which check no operand themselves, refuse host tensors before the library is called:
+    their addresses mean nothing to a kernel."""
+    called = []
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda i: 0)
+    monkeypatch.setattr(ops, "call", lambda *a: called.append(a))
+    a, w = torch.zeros(4, 64, dtype=torch.bfloat16), torch.zeros(8, 64, dtype=torch.bfloat16)
+    out, meta = torch.zeros(4, 8, dtype=torch.bfloat16), torch.zeros(4, device="meta")
+    for f in (lambda: ops.gemm(a, w, None, out), lambda: ops.gemm(a, w, None, out, ws=torch.zeros(64)),
+              lambda: ops.rowop(out, partials=torch.zeros(1, 4, 8)), lambda: ops._stream(meta)):
+        with pytest.raises(ValueError):
+            f()
+    assert not called
