@@ -300,3 +300,27 @@ def _load_fresh(path):
         return _capi.load(path)
     finally:
         _capi._lib = saved
+
+
+def test_conv3x3_validation(lib):
+    """Every refusal of fam_conv3x3, from a descriptor it takes up to its launch (no field of which is wrong)."""
+    def rc(H=16, W=16, Cn=64, stride=1, ws=None, wsf=0, **kw):
+        d = _capi.GemmDesc(4096, 64, 4096, 576, 4096, 4096, 64, 256, 64, 576)
+        d.rows_per_batch, d.gate_ns = 256, 1
+        for k, v in kw.items():
+            setattr(d, k, v)
+        return lib.fam_conv3x3(C.byref(d), H, W, Cn, stride, ws, wsf, None)
+    bad, no = _capi.FAM_ERR_INVALID_ARG, _capi.FAM_ERR_UNSUPPORTED
+    assert lib.fam_conv3x3(None, 16, 16, 64, 1, None, 0, None) == bad
+    assert rc(a=None) == bad and rc(w=None) == bad and rc(out=None) == bad
+    assert rc(ws=4096 + 8, wsf=1 << 20) == bad and rc(wsf=1 << 20) == bad and rc(wsf=-1) == bad     # workspace
+    assert rc(stride=3) == bad and rc(stride=0) == bad and rc(H=32, W=31, stride=2, M=16 * 15) == bad
+    assert rc(H=15) == bad and rc(M=255) == bad and rc(H=-16, W=-16) == bad and rc(H=1 << 24, W=1, M=1 << 24) == bad
+    assert rc(Cn=60, K=576) == bad and rc(Cn=72) == bad and rc(Cn=56) == bad and rc(K=640, ldw=640) == bad   # K = 9 C rounded up
+    assert rc(lda=56) == bad and rc(lda=68) == bad and rc(ldw=568) == bad and rc(ldo=60) == bad and rc(N=0) == bad
+    assert rc(a=4096 + 8) == bad and rc(w=4096 + 8) == bad
+    assert rc(act=99) == bad and rc(rows_per_batch=0) == bad and rc(gate=4096) == bad               # a gate needs a residual
+    assert rc(H=8, W=15, M=120) == no and rc(N=62) == no and rc(ldo=66) == no                       # big-kernel limits
+    assert rc(bias=4096 + 2) == no and rc(out=4096 + 4) == no and rc(prologue=_capi.FAM_PRO_LAYERNORM) == no
+    assert rc(res=4096, ldr=66) == no and rc(res=4096, ldr=64, gate=4096, gate_ns=2) == no
+    assert rc(H=16384, W=16384, M=1 << 28) == no                                                    # 2 GiB

@@ -1047,13 +1047,17 @@ def test_gemm_rows_past_the_end_read_as_zero(M, N, K):
 
 
 @pytest.mark.parametrize("M,N,K", [(1, 16, 64), (16, 33, 256), (17, 1024, 1024), (32, 1003, 768), (33, 48, 512),
-                                   (64, 1030, 1024), (32, 1024, 4096), (17, 1024, 3072), (31, 520, 1088), (5, 7, 192)])
+                                   (64, 1030, 1024), (32, 1024, 4096), (17, 1024, 3072), (31, 520, 1088), (5, 7, 192),
+                                   (16, 1024, 1024), (9, 1024, 2048), (7, 1024, 4096), (24, 1026, 2048), (45, 1026, 2048),
+                                   (64, 1024, 4096), (16, 40, 512), (9, 40, 768), (12, 33, 1280), (16, 40, 1536),
+                                   (20, 40, 256), (24, 40, 384), (50, 40, 192), (40, 40, 768)])
 def test_staged_panels_small_m(M, N, K):
-    """fam_gemm_partial, fam_gemm_final and the skinny fam_gemm at <= 64 rows, whose operands reach the MFMAs through LDS panels
-    of 64, 128 or 256 columns per wave: rows and columns that do not fill a 16-row tile, K that leaves waves
-    without a range (768, 192), K outside the panels (1088: the register form), row pitches wider than K with
-    NaN around the operands (a read outside them would show).  fp32 sums of exact bf16 products: within
-    K 2^-23 sum |a| |w| of float64 in any order; the bf16 result adds half an ulp (2^-9)."""
+    """fam_gemm_partial, fam_gemm_final and the skinny fam_gemm at <= 64 rows, whose operands reach the MFMAs
+    through LDS panels of 64, 128, 192 or 256 columns per wave, each width with 16, 32 and 64 rows: rows and
+    columns that do not fill a 16-row tile, K that leaves waves without a range (768, 192), K outside the panels
+    (1088: the register form), row pitches wider than K with NaN around the operands (a read outside them would
+    show).  fp32 sums of exact bf16 products: within K 2^-23 sum |a| |w| of float64 in any order; the bf16 result
+    adds half an ulp (2^-9)."""
     a = torch.full((M + 16, K + 64), float("nan"), dtype=torch.bfloat16)
     w = torch.full((N + 16, K + 64), float("nan"), dtype=torch.bfloat16)
     a[:M, :K], w[:N, :K] = rnd(M, K, seed=171), rnd(N, K, seed=172, scale=0.02)
@@ -1063,10 +1067,9 @@ def test_staged_panels_small_m(M, N, K):
     lim = K * 2.0 ** -23 * (a[:M, :K].double().abs() @ w[:N, :K].double().abs().t())
     part, S = ops().gemm_partial(ad, wd)
     assert ((part.double().sum(0).cpu() - ref).abs() <= lim).all()
-    if N % 4 == 0:
-        o32 = torch.empty(M, N, dtype=torch.float32, device="cuda")
-        ops().gemm(ad, wd, None, o32, out_f32=True)
-        assert ((o32.double().cpu() - ref).abs() <= lim).all()
+    o32 = torch.empty(M, N, dtype=torch.float32, device="cuda")
+    ops().gemm(ad, wd, None, o32, out_f32=True)
+    assert ((o32.double().cpu() - ref).abs() <= lim).all()
     if K <= 4096:
         y, ss = ops().gemm_final(ad, wd, dev(b), want_sumsq=True)
         y = y.double().cpu()

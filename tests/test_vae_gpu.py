@@ -47,7 +47,7 @@ def test_im2col3x3(H, W, C, stride):
 
 
 # Edges of the image on every side of a tile, C below, off and above the 64-wide K block, both
-# strides, padded rows, and image sizes that reach each tile of the product and its split planes.
+# strides, padded rows (every tile of the product: test_conv3x3_on_every_tile).
 @pytest.mark.parametrize("H,W,C,N,stride,ldx", [
     (9, 17, 8, 12, 1, 8), (1, 130, 24, 64, 1, 32), (130, 1, 64, 20, 1, 64), (28, 56, 40, 100, 2, 48),
     (16, 20, 160, 96, 1, 160), (14, 28, 640, 640, 1, 640), (56, 112, 320, 640, 2, 320), (96, 96, 80, 256, 1, 80),
@@ -89,6 +89,73 @@ def test_conv3x3_equals_im2col_gemm(H, W, C, N, stride, ldx):
     img = F.pad(img, (1, 1, 1, 1)) if stride == 1 else F.pad(img, (0, 1, 0, 1))
     ref = F.conv2d(img, k, bias.float().cpu(), stride=stride).reshape(N, P).t() + res.float().cpu()
     assert _rel(outs[1], ref) <= 1e-2
+
+
+def _conv_and_gemm(H, W, C, N, act=0, gate=False, f32=False):
+    """fam_conv3x3 of an H x W image and fam_gemm_ws of its neighbourhoods: (conv, gemm, rows, w, bias, res, gate)."""
+    from fam import _capi
+    import ctypes
+    lib, P, kp = _lib(), H * W, (9 * C + 63) // 64 * 64
+    g = torch.Generator().manual_seed(H * 131 + C)
+    rn = lambda *s: torch.randn(*s, generator=g).to(BF)
+    x, w = rn(P, C).cuda(), torch.zeros(N, kp, dtype=BF)
+    w[:, :9 * C] = rn(N, 9 * C) / math.sqrt(9 * C)
+    w, bias, res, gt = w.cuda(), rn(N).cuda(), rn(P, N).cuda(), rn(2, N).cuda()
+    res = res.float() if f32 else res
+    rows = torch.empty(P, kp, dtype=BF, device="cuda")
+    assert lib.fam_im2col3x3(x.data_ptr(), C, H, W, C, 1, rows.data_ptr(), kp, kp, _s()) == 0
+    wsf = lib.fam_gemm_ws_floats(P, N, kp)
+    ws = torch.empty(max(wsf, 4), device="cuda")
+    outs = []
+    for conv in (True, False):
+        y = torch.empty(P, N, dtype=torch.float32 if f32 else BF, device="cuda")
+        a = x if conv else rows
+        d = _capi.GemmDesc(a.data_ptr(), a.stride(0), w.data_ptr(), kp, bias.data_ptr(), y.data_ptr(), N, P, N, kp)
+        d.act, d.res, d.ldr, d.rows_per_batch, d.gate_ns, d.out_f32 = act, res.data_ptr(), N, (P + 1) // 2, 1, int(f32)
+        if gate:
+            d.gate, d.gate_bs = gt.data_ptr(), N
+        if conv:
+            assert lib.fam_conv3x3(ctypes.byref(d), H, W, C, 1, ws.data_ptr(), wsf, _s()) == 0, lib.fam_last_error()
+        else:
+            assert lib.fam_gemm_ws(ctypes.byref(d), ws.data_ptr(), wsf, _s()) == 0, lib.fam_last_error()
+        outs.append(y)
+    return (*outs, rows, w, bias, res, gt)
+
+
+# A shape for every tile the library's plan can choose on 256 CUs, for channels that are (second
+# half) and are not (first) whole K blocks: 64 x 64 with four and two K slots, 128 x 96, 128 x 128
+# with one and two K groups, 224 x 256, 256 x 256, and K splits of the 64, 128, 224 and 256 tiles.
+@pytest.mark.parametrize("H,W,C,N", [
+    (10, 16, 88, 20), (56, 56, 88, 768), (75, 100, 88, 640), (56, 56, 200, 768), (56, 56, 264, 768), (75, 100, 88, 1280),
+    (75, 100, 88, 2048), (10, 16, 296, 20), (28, 28, 600, 1280), (64, 64, 720, 768), (64, 64, 1000, 1280),
+    (16, 16, 64, 64), (56, 56, 64, 768), (190, 200, 64, 64), (190, 200, 64, 128), (56, 56, 256, 768), (112, 224, 64, 320),
+    (75, 100, 64, 2048), (16, 16, 320, 64), (28, 28, 640, 1280), (100, 125, 640, 192), (64, 64, 1024, 1280)])
+def test_conv3x3_on_every_tile(H, W, C, N):
+    """The bits of the product on the laid-out neighbourhoods, and its value: fp32 accumulation, half a bf16
+    ulp (2^-8 of the value at most) of the product with its bias and of the sum with the residual."""
+    y, ref, rows, w, bias, res, _ = _conv_and_gemm(H, W, C, N)
+    assert torch.equal(y, ref)
+    v = rows.float() @ w.float().t() + bias.float()
+    exact = v + res.float()
+    assert ((y.float() - exact).abs() <= 2.0 ** -8 * (v.abs() + exact.abs()) + 1e-4).all()
+
+
+@pytest.mark.parametrize("H,W,C,N", [(20, 24, 24, 100), (14, 28, 640, 640), (56, 56, 264, 768)])
+@pytest.mark.parametrize("act,gate,f32", [("FAM_ACT_GELU_TANH", False, False), ("FAM_ACT_SILU", True, False),
+                                          ("FAM_ACT_NONE", True, True), ("FAM_ACT_RELU", False, True)])
+def test_conv3x3_epilogues(H, W, C, N, act, gate, f32):
+    """Activation, a gate row per half of the pixels, and fp32 residual and output, whole and split K.  The
+    product with its bias is rounded to bf16 (2^-8 of it at most) before the activation, whose slope is at
+    most 1.13, and the gate; then the sum."""
+    from fam import _capi
+    y, ref, rows, w, bias, res, gt = _conv_and_gemm(H, W, C, N, getattr(_capi, act), gate, f32)
+    assert torch.equal(y, ref)
+    v = rows.float() @ w.float().t() + bias.float()
+    f = {"FAM_ACT_GELU_TANH": lambda t: F.gelu(t, approximate="tanh"), "FAM_ACT_SILU": F.silu, "FAM_ACT_RELU": F.relu,
+         "FAM_ACT_NONE": lambda t: t}[act]
+    gated = gt.float()[torch.arange(H * W, device="cuda") // ((H * W + 1) // 2)] if gate else torch.ones_like(v)
+    exact = res.float() + gated * f(v)
+    assert ((y.float() - exact).abs() <= 2.0 ** -8 * (1.13 * (gated * v).abs() + exact.abs()) + 1e-4).all()
 
 
 def test_vae_patch_im2col():
