@@ -1180,7 +1180,9 @@ __global__ __launch_bounds__(256) void attn_cross_kernel(AttnArgs a) {
 // exact as attn_tiled_kernel's, which these masks ran on before: an exact running max and a sum of
 // the rounded probabilities, with the first tile in halves.  1592 x 1592 joint mask, 24 x 128
 // heads: 273 us there, 64 here (61 with the lazy max below); error against float64 2.218e-3 there,
-// 2.217e-3 here, 2.334e-3 with the lazy max (peaked scores, x 5: 1.71, 1.69 and 1.94e-3).
+// 2.217e-3 here, 2.334e-3 with the lazy max (peaked scores, x 5: 1.71, 1.69 and 1.94e-3).  Masks
+// without a clear tile (half of the entries at random): 24 x 128 heads of 1560 x 1560 267 -> 74 us, 16
+// x 64 of 700 x 700 57 -> 20, one 128-wide head of 129 x 300 35 -> 16.
 // KW = 2 (head dim 128, a grid of at most one workgroup per CU): 8 waves in two key groups of
 // 4; group g takes the tiles g, g + 2, g + 4, ... of the same 128 queries with its own LDS slots,
 // so each SIMD runs two waves (one's softmax under the other's MFMAs) although the grid leaves

@@ -214,10 +214,10 @@ __device__ __forceinline__ void row_stats(const GemmArgs& g, int64_t m0, int row
 // weights in HBM, 4.5 us with everything in L2, 1.8 us for a kernel that only loads and stores).
 // A staged wave fetches the KW-wide k range that it alone uses, of every row, with direct-to-LDS
 // buffer loads instead: one load is 1 KB = 512 / KW rows of KW contiguous values.  Nothing is
-// shared between waves, so the wave's own vmcnt wait is all the synchronisation there is before
-// its products.  The 16-byte chunk c of row r sits at c ^ panel_swz(r) (lane j fetches the chunk
+// shared between waves (but in one form of skinny_staged_kernel), so the wave's own vmcnt wait is
+// all the synchronisation there is before its products.  The 16-byte chunk c of row r sits at c ^ panel_swz(r) (lane j fetches the chunk
 // that belongs in its slot), which makes the fragment reads of 16 rows hit 16 distinct bank
-// groups.  Rows past M or N are past the descriptor's range and read zeros.
+// groups.  Rows past M or N that are fetched are past the descriptor's range and read zeros.
 template <int KW>
 __device__ __forceinline__ int panel_swz(int r) { return KW == 64 || KW == 192 ? (r >> 1) & 7 : r & 15; }
 
@@ -486,8 +486,9 @@ __global__ __launch_bounds__(NW * 64) void skinny_kernel(GemmArgs g) {
 // staged panels, NW waves staging KW columns of K each (a multiple of KW).  The row sums of the
 // folded form come from the fragments the MFMAs use; it takes 8 waves, so that a SIMD's two waves
 // share them, the plain form 4, or 8 for 16 rows of K up to 2048.  The DiT4DiT head (17 rows,
-// K = 768, about 50 such launches a step): 2100 -> 1943 us for a call of 4
-// steps.
+// K = 768, about 50 such launches a step): 2100 -> 1940 us for a call of 4 steps.  N = K = 1024,
+// plain / folded: 16 rows 4.5 -> 3.5 / 4.8 -> 4.3 us, 32 rows 5.8 -> 4.0 / 7.0 -> 5.2, 64 rows 7.7 ->
+// 6.0 / 10.4 -> 8.2.
 // The sums keep skinny_kernel's grouping, and so its bits: NG runs of G k-steps (its waves' shares
 // of K), each an accumulator of its own, added in order.  Where a wave's runs are not its own panel
 // (the folded form's K = 768 is 8 runs of 3 k-steps and 6 panels of 4), the panels are shared behind
@@ -714,7 +715,7 @@ __global__ __launch_bounds__(256) void partial_kernel(PartArgs g) {
 // partial_staged_kernel: partial_kernel's split (16 columns x 4 KW of K per workgroup, the same
 // planes) with staged panels.  K is a multiple of KW: a wave's range lies in K or past it.
 // Measured at M = 32, N = 1024 (graph-timed, weights from HBM): K = 1024 in 4 planes 2.7 -> 2.4
-// us, K = 4096 in 4 planes 5.3 -> 4.15 us.
+// us, K = 4096 in 4 planes 5.3 -> 4.15 us (64 rows 7.4 -> 5.35).
 template <int MT, int KW>
 __global__ __launch_bounds__(256) void partial_staged_kernel(PartArgs g) {
   constexpr bool WD = MT == 4 && KW == 256;   // 4 x 80 rows x 512 B would be the whole LDS
@@ -1059,10 +1060,11 @@ __global__ __launch_bounds__(NW * 64) void final_kernel(FinalArgs g) {
 }
 
 // final_staged_kernel: the same workgroup (16 columns, whole K, 4 waves) with staged panels, for
-// K <= 1024, a multiple of KW.  Graph-timed at M = 32, K = 1024 with the weights in HBM: N = 1024
-// 4.8 -> 3.35 us, 3072 5.3 -> 4.15 us, 4096 + GELU 5.6 -> 4.6 us.  A workgroup holds up to 96 KB of
-// LDS (M <= 32; 128 KB at 64 rows), so one runs per CU: also above 256 workgroups ahead of the
-// register form (N = 9216: 10.8 -> 9.1 us for the bare product).
+// 128 < K <= 1024, a multiple of KW.  Graph-timed at M = 32, K = 1024 with the weights in HBM: N =
+// 1024 4.8 -> 3.35 us, 3072 5.3 -> 4.15 us, 4096 + GELU 5.6 -> 4.6 us; 64 rows (weights straight to
+// registers) N = 1024 7.3 -> 5.2 us, 14336 21.7 -> 18.0.  A workgroup holds up to 96 KB of LDS (M <=
+// 32; 128 KB at 64 rows), so one runs per CU, and above 512 workgroups tiles that are mostly padding
+// stay on the register form (staged_crowded).
 template <int MT, int KW>
 __global__ __launch_bounds__(256) void final_staged_kernel(FinalArgs g) {
   constexpr bool WD = MT == 4 && KW == 256;

@@ -36,12 +36,17 @@ from collections import OrderedDict
 from typing import Dict, Optional, Tuple
 
 import torch
+from torch.autograd import forward_ad
 
 from . import _capi
 from ._capi import call
 
 _BF16 = torch.bfloat16
 _PLAIN_TYPES = (torch.Tensor, torch.nn.Parameter)
+# what _plain asks on every call, looked up once
+_dispatch_modes, _function_modes = torch._C._len_torch_dispatch_stack, torch._C._len_torch_function_stack
+_transform, _jit_trace = torch._C._functorch.peek_interpreter_stack, torch._C._get_tracing_state
+_profiling = torch._C._autograd._profiler_enabled
 
 
 def _stream(t: torch.Tensor) -> int:
@@ -58,8 +63,8 @@ def _plain(*tensors) -> bool:
     tensors, export), a functorch transform (vmap, grad, jvp), forward-mode duals, a gradient to
     record, the profiler.  Then the operator would do nothing but call its implementation, and the
     wrappers below call it themselves: the dispatcher's way through a Python operator costs a call
-    5 us (ops.linear at 32 rows 17.8 -> 8.5 us a call with the views and checks it no longer makes,
-    adaln_forward 20.4 -> 10.6 us; the kernels take 4 and 7 us)."""
+    5 us (ops.linear at 32 rows 17.9 -> 8.9 us a call with the views and checks it no longer makes,
+    adaln_forward 20.5 -> 10.6 us; the kernels take 4 and 7 us)."""
     if torch.compiler.is_compiling():
         return False
     grad = torch.is_grad_enabled()
@@ -67,10 +72,8 @@ def _plain(*tensors) -> bool:
         if t is not None and (type(t) not in _PLAIN_TYPES or (grad and t.requires_grad) or t.is_conj() or t.is_neg()
                               or t._is_zerotensor()):
             return False
-    return not (torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
-                or torch._C._functorch.peek_interpreter_stack() is not None
-                or torch.autograd.forward_ad._current_level >= 0 or torch._C._get_tracing_state() is not None
-                or torch._C._autograd._profiler_enabled())
+    return not (_dispatch_modes() or _function_modes() or _transform() is not None or forward_ad._current_level >= 0
+                or _jit_trace() is not None or _profiling())
 
 
 def _check(t: torch.Tensor, name: str, dtype=_BF16, device: bool = True) -> None:
